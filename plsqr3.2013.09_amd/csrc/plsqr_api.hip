@@ -418,26 +418,78 @@ int launch_cols(plsqr_op *op, const double *u, double *v, const Scal *sc, double
     return PLSQR_OK;
 }
 
+// Segments per wavefront of the exact-order sums: as many as fill a round of
+// EXACT_CH products at their mean length.
+int exact_seg(long long nnz, int segs) {
+    const long long mean = nnz / std::max(segs, 1);
+    return mean >= 64 ? 4 : mean >= 16 ? 16 : 64;
+}
+
+// y += A x on the CSR in the reference's order
+int launch_rows_exact(plsqr_op *op, const double *x, double *y, const Scal *sc) {
+    using namespace plsqr;
+    const int seg = exact_seg(op->nnz_k, op->m_k);
+    const int gk = grid_for(op->m_k, seg * (256 / kWave), op->cu * 8);
+    const int gd = op->m_d > 0 ? grid_for(op->m_d, 256, op->cu * 4) : 0;
+#define ROWS_EXACT(SEG)                                                                                        \
+    hipLaunchKernelGGL((k_rows_exact<SEG>), dim3(gk + gd), dim3(256), 0, op->stream, op->m_k, op->m, gk, op->rp, \
+                       op->ci, op->rv, x, y, sc)
+    if (seg == 4)
+        ROWS_EXACT(4);
+    else if (seg == 16)
+        ROWS_EXACT(16);
+    else
+        ROWS_EXACT(64);
+#undef ROWS_EXACT
+    LAUNCH_CHECK(op);
+    return PLSQR_OK;
+}
+
+// v += A^T u on the kernel CSC and the damping CSC in the reference's order
+int launch_cols_exact(plsqr_op *op, const double *u, double *v, const Scal *sc) {
+    using namespace plsqr;
+    const int seg = exact_seg(op->nnz_k, op->n);
+    const dim3 g(grid_for(op->n, seg * (256 / kWave), op->cu * 8));
+#define COLS_EXACT(SEG)                                                                                      \
+    hipLaunchKernelGGL((k_cols_exact<SEG>), g, dim3(256), 0, op->stream, op->n, op->m_k, op->kcp, op->kri,     \
+                       op->kv, op->dcp, op->dri, op->dcv, u, sc, v)
+    if (seg == 4)
+        COLS_EXACT(4);
+    else if (seg == 16)
+        COLS_EXACT(16);
+    else
+        COLS_EXACT(64);
+#undef COLS_EXACT
+    LAUNCH_CHECK(op);
+    return PLSQR_OK;
+}
+
+// the two halves of ||u|| (kernel rows, damping rows) side by side, and ||v||
+int launch_norms_exact(plsqr_op *op, const Scal *sc) {
+    using namespace plsqr;
+    hipLaunchKernelGGL(k_dnrm2_seq, dim3(2), dim3(128), 0, op->stream, SeqVec{op->m_k, op->u, &op->sc->pk},
+                       SeqVec{op->m_d, op->u + op->m_k, &op->sc->pd}, sc, 0);
+    LAUNCH_CHECK(op);
+    return PLSQR_OK;
+}
+
+int launch_vnorm_exact(plsqr_op *op) {
+    using namespace plsqr;
+    const SeqVec v{op->n, op->v, &op->sc->pv};
+    hipLaunchKernelGGL(k_dnrm2_seq, dim3(1), dim3(128), 0, op->stream, v, v, (const Scal *)op->sc, 1);
+    LAUNCH_CHECK(op);
+    return PLSQR_OK;
+}
+
 // y += A x  (mode 1) on device pointers
 int aprod1_dev(plsqr_op *op, const double *x, double *y) {
-    if (op->exact) {
-        hipLaunchKernelGGL(plsqr::k_rows_exact, dim3(grid_for(op->m, BS, op->cu * 8)), dim3(BS), 0, op->stream,
-                           op->m, op->rp, op->ci, op->rv, x, y, (const Scal *)nullptr);
-        LAUNCH_CHECK(op);
-        return PLSQR_OK;
-    }
+    if (op->exact) return launch_rows_exact(op, x, y, nullptr);
     return launch_rows(op, x, y, nullptr, nullptr);
 }
 
 // x += A^T y  (mode 2) on device pointers
 int aprod2_dev(plsqr_op *op, double *x, const double *y) {
-    if (op->exact) {
-        hipLaunchKernelGGL(plsqr::k_cols_exact, dim3(grid_for(op->n, BS, op->cu * 8)), dim3(BS), 0, op->stream,
-                           op->n, op->m_k, op->kcp, op->kri, op->kv, op->dcp, op->dri, op->dcv, y,
-                           (const Scal *)nullptr, x);
-        LAUNCH_CHECK(op);
-        return PLSQR_OK;
-    }
+    if (op->exact) return launch_cols_exact(op, y, x, nullptr);
     return launch_cols(op, y, x, nullptr, nullptr);
 }
 
@@ -1494,24 +1546,12 @@ static int enqueue_iteration(plsqr_op *op, double *x, double *w, double *se, dou
     using namespace plsqr;
     int rc;
     if (op->exact) {
-        hipLaunchKernelGGL(k_rows_exact, dim3(grid_for(op->m, BS, op->cu * 8)), dim3(BS), 0, op->stream, op->m, op->rp,
-                           op->ci, op->rv, op->v, op->u, (const Scal *)op->sc);
-        LAUNCH_CHECK(op);
-        hipLaunchKernelGGL(k_dnrm2_seq, dim3(1), dim3(64), 0, op->stream, op->m_k, op->u, &op->sc->pk,
-                           (const Scal *)op->sc, 0);
-        hipLaunchKernelGGL(k_dnrm2_seq, dim3(1), dim3(64), 0, op->stream, op->m_d, op->u + op->m_k, &op->sc->pd,
-                           (const Scal *)op->sc, 0);
-        LAUNCH_CHECK(op);
+        if ((rc = launch_rows_exact(op, op->v, op->u, op->sc)) || (rc = launch_norms_exact(op, op->sc))) return rc;
         hipLaunchKernelGGL(k_s_beta, dim3(1), dim3(256), 0, op->stream, op->sc, op->part, 0);
         LAUNCH_CHECK(op);
-        hipLaunchKernelGGL(k_cols_exact, dim3(grid_for(op->n, BS, op->cu * 8)), dim3(BS), 0, op->stream, op->n,
-                           op->m_k, op->kcp, op->kri, op->kv, op->dcp, op->dri, op->dcv, op->u, (const Scal *)op->sc,
-                           op->v);
-        hipLaunchKernelGGL(k_dnrm2_seq, dim3(1), dim3(64), 0, op->stream, op->n, op->v, &op->sc->pv,
-                           (const Scal *)op->sc, 1);
-        LAUNCH_CHECK(op);
+        if ((rc = launch_cols_exact(op, op->u, op->v, op->sc)) || (rc = launch_vnorm_exact(op))) return rc;
         hipLaunchKernelGGL(k_s_alpha, dim3(1), dim3(256), 0, op->stream, op->sc, op->part, 0);
-        hipLaunchKernelGGL(k_dknorm_seq, dim3(1), dim3(64), 0, op->stream, op->n, w, op->sc);
+        hipLaunchKernelGGL(k_dknorm_seq, dim3(1), dim3(128), 0, op->stream, op->n, w, op->sc);
         hipLaunchKernelGGL((k_update<BS>), dim3(op->G6), dim3(BS), 0, op->stream, op->n, (const Scal *)op->sc, op->v,
                            w, x, se, (double *)nullptr);
         LAUNCH_CHECK(op);
@@ -1575,11 +1615,7 @@ static int solve_fp64(plsqr_op *op, const double *b_dev, const plsqr_solve_opts 
     LAUNCH_CHECK(op);
     // beta = ||u||
     if (op->exact) {
-        hipLaunchKernelGGL(k_dnrm2_seq, dim3(1), dim3(64), 0, op->stream, op->m_k, op->u, &op->sc->pk,
-                           (const Scal *)nullptr, 0);
-        hipLaunchKernelGGL(k_dnrm2_seq, dim3(1), dim3(64), 0, op->stream, op->m_d, op->u + op->m_k, &op->sc->pd,
-                           (const Scal *)nullptr, 0);
-        LAUNCH_CHECK(op);
+        if ((rc = launch_norms_exact(op, nullptr))) return rc;
         hipLaunchKernelGGL(k_s_init_beta, dim3(1), dim3(256), 0, op->stream, op->sc, op->part, 0);
     } else {
         // partials laid out as [kernel, damping] pairs, like k_rows
@@ -1591,12 +1627,7 @@ static int solve_fp64(plsqr_op *op, const double *b_dev, const plsqr_solve_opts 
     LAUNCH_CHECK(op);
     // v = A^T u (scaled by 1/beta on the fly), alpha
     if (op->exact) {
-        hipLaunchKernelGGL(k_cols_exact, dim3(grid_for(op->n, BS, op->cu * 8)), dim3(BS), 0, op->stream, op->n,
-                           op->m_k, op->kcp, op->kri, op->kv, op->dcp, op->dri, op->dcv, op->u, (const Scal *)op->sc,
-                           op->v);
-        hipLaunchKernelGGL(k_dnrm2_seq, dim3(1), dim3(64), 0, op->stream, op->n, op->v, &op->sc->pv,
-                           (const Scal *)op->sc, 1);
-        LAUNCH_CHECK(op);
+        if ((rc = launch_cols_exact(op, op->u, op->v, op->sc)) || (rc = launch_vnorm_exact(op))) return rc;
         hipLaunchKernelGGL(k_s_init_alpha, dim3(1), dim3(256), 0, op->stream, op->sc, op->part, 0, trace_d);
     } else {
         hipLaunchKernelGGL(k_fill, dim3(grid_for(op->part_len, 256, 64)), dim3(256), 0, op->stream,

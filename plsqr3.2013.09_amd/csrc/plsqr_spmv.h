@@ -14,7 +14,7 @@
 //                    that slice stays resident in the XCD's 4 MB L2.  The S
 //                    per-slice column sums are combined in a fixed order with the
 //                    damping column sums (one lane per column, rows ascending).
-// Exact-order kernels: one lane per row / column, summed sequentially in the
+// Exact-order kernels: every row / column summed sequentially in the
 //                    reference's order (CPUSpMV.c:50-89,162-183,203-245,255-296).
 #include "plsqr_kernels.h"
 
@@ -301,16 +301,67 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_combine(int m_k, int m, int S
     }
 }
 
-// Exact order: one lane per row, sequential sum from 0 in ascending column
-// order.  For a kernel row this is the sequence of partial sums the CSC
-// scatter cpuSpMV_CSC (CPUSpMV.c:171-180) builds in tmp[r]; for a damping row
-// it is cpuSpMV_CSR_v2 (CPUSpMV.c:75-84).
-__global__ __launch_bounds__(256) void k_rows_exact(int m, const int *__restrict__ rp,
-                                                    const int *__restrict__ ci,
-                                                    const double *__restrict__ av,
-                                                    const double *__restrict__ x,
-                                                    double *__restrict__ y,
+// ---------------------------------------------------------------------------
+// Exact order
+// ---------------------------------------------------------------------------
+// One wavefront adds SEG consecutive segments (rows of the CSR, columns of the
+// CSC), each sequentially from 0 in storage order, lane l < SEG owning segment
+// s0 + l.  What bounds it is the serial chain of one segment; a lane walking
+// its segment in global memory (one uncoalesced value, index and gather per
+// addition) paid a memory latency per entry.  Here the segments' entries, one
+// contiguous range, are multiplied EXACT_CH at a time by all 64 lanes with
+// coalesced loads and the products left in LDS, so a lane's additions wait for
+// LDS only.  SEG follows the mean segment length (exact_seg), so that a round
+// of EXACT_CH products covers the wavefront's segments: 24^3 / 60k rays, 170
+// entries per column: 349 us by one lane per column, 61 us here.
+constexpr int EXACT_CH = 512;
+
+template <int SEG, class F>
+__device__ __forceinline__ double segments_exact(int s0, int ns, const int *__restrict__ ptr, double *buf, F product) {
+    static_assert(SEG <= kWave && EXACT_CH % kWave == 0, "one segment per lane, whole rounds");
+    const int lane = threadIdx.x % kWave;
+    const bool own = lane < SEG && s0 + lane < ns;
+    const int beg = own ? ptr[s0 + lane] : 0, end = own ? ptr[s0 + lane + 1] : 0;
+    const int first = ptr[s0], last = ptr[min(s0 + SEG, ns)];
+    double acc = 0.0;
+    for (int q0 = first, cnt; q0 < last; q0 += cnt) {
+        cnt = min(EXACT_CH, last - q0);
+#pragma unroll
+        for (int j = 0; j < EXACT_CH / kWave; ++j) {
+            const int k = j * kWave + lane;
+            if (k < cnt) buf[k] = product(q0 + k);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        int k = max(beg - q0, 0);
+        const int e = min(end - q0, cnt);
+        for (; k + 3 < e; k += 4) {
+            const double p0 = buf[k], p1 = buf[k + 1], p2 = buf[k + 2], p3 = buf[k + 3];
+            acc += p0;
+            acc += p1;
+            acc += p2;
+            acc += p3;
+        }
+        for (; k < e; ++k) acc += buf[k];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    return acc;
+}
+
+// Rows summed sequentially from 0 in ascending column order: for a kernel row
+// the sequence of partial sums the CSC scatter cpuSpMV_CSC
+// (CPUSpMV.c:171-180) builds in tmp[r]; for a damping row cpuSpMV_CSR_v2
+// (CPUSpMV.c:75-84).  Workgroups below gk take kernel rows by wavefronts, the
+// others damping rows (1 to 4 entries each) one per lane.
+template <int SEG>
+__global__ __launch_bounds__(256) void k_rows_exact(int m_k, int m, int gk, const int *__restrict__ rp,
+                                                    const int *__restrict__ ci, const double *__restrict__ av,
+                                                    const double *__restrict__ x, double *__restrict__ y,
                                                     const Scal *__restrict__ sc) {
+    __shared__ double buf[256 / kWave][EXACT_CH];
     double s1 = 1.0, s2 = 1.0;
     const bool scaled = sc != nullptr;
     if (scaled) {
@@ -318,13 +369,23 @@ __global__ __launch_bounds__(256) void k_rows_exact(int m, const int *__restrict
         s1 = sc->ib;
         s2 = -sc->alpha;
     }
-    for (long long r = (long long)blockIdx.x * 256 + threadIdx.x; r < m; r += (long long)gridDim.x * 256) {
-        double acc = 0.0;
-        for (int k = rp[r]; k < rp[r + 1]; ++k) acc += av[k] * x[ci[k]];
+    auto store = [&](long long r, double acc) {
         double yn = y[r];
         if (scaled) yn = (yn * s1) * s2;
         y[r] = yn + acc;
+    };
+    if ((int)blockIdx.x < gk) {
+        const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+        const int nw = gk * (256 / kWave);
+        for (long long s0 = ((long long)blockIdx.x * (256 / kWave) + wv) * SEG; s0 < m_k; s0 += (long long)nw * SEG) {
+            const double acc = segments_exact<SEG>((int)s0, m_k, rp, buf[wv], [&](int k) { return av[k] * x[ci[k]]; });
+            if (lane < SEG && s0 + lane < m_k) store(s0 + lane, acc);
+        }
+        return;
     }
+    for (long long r = (long long)m_k + (long long)(blockIdx.x - gk) * 256 + threadIdx.x; r < m;
+         r += (long long)(gridDim.x - gk) * 256)
+        store(r, damp_row_sum(rp[r], rp[r + 1], ci, av, x));
 }
 
 // ---------------------------------------------------------------------------
@@ -710,7 +771,8 @@ __global__ __launch_bounds__(BS) void k_cols_combine(int n, int m_k, int nsl,
 }
 
 // Exact order (cpuSpMVTranspose_CSC and _v2, CPUSpMV.c:230-240,281-291, and
-// aprod_impl.c:487-489): one lane per column.
+// aprod_impl.c:487-489): SEG columns per wavefront.
+template <int SEG>
 __global__ __launch_bounds__(256) void k_cols_exact(int n, int m_k, const int *__restrict__ cp,
                                                     const int *__restrict__ ri,
                                                     const double *__restrict__ av,
@@ -720,6 +782,7 @@ __global__ __launch_bounds__(256) void k_cols_exact(int n, int m_k, const int *_
                                                     const double *__restrict__ u,
                                                     const Scal *__restrict__ sc,
                                                     double *__restrict__ v) {
+    __shared__ double buf[256 / kWave][EXACT_CH];
     double ib = 1.0, vs = 1.0;
     const bool scaled = sc != nullptr;
     if (scaled) {
@@ -728,14 +791,18 @@ __global__ __launch_bounds__(256) void k_cols_exact(int n, int m_k, const int *_
         vs = sc->vscale;
     }
     const double *ud = u + m_k;
-    for (int c = blockIdx.x * 256 + threadIdx.x; c < n; c += gridDim.x * 256) {
-        double tk = 0.0;
-        for (int k = cp[c]; k < cp[c + 1]; ++k) tk += av[k] * (u[ri[k]] * ib);
-        double td = 0.0;
-        for (int k = dcp[c]; k < dcp[c + 1]; ++k) td += dav[k] * (ud[dri[k]] * ib);
-        double vn = v[c];
-        if (scaled) vn = vn * vs;
-        v[c] = vn + (tk + td);
+    const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int nw = gridDim.x * (256 / kWave);
+    for (long long s0 = ((long long)blockIdx.x * (256 / kWave) + wv) * SEG; s0 < n; s0 += (long long)nw * SEG) {
+        const double tk = segments_exact<SEG>((int)s0, n, cp, buf[wv], [&](int k) { return av[k] * (u[ri[k]] * ib); });
+        const int c = (int)s0 + lane;
+        if (lane < SEG && c < n) {
+            double td = 0.0;
+            for (int k = dcp[c]; k < dcp[c + 1]; ++k) td += dav[k] * (ud[dri[k]] * ib);
+            double vn = v[c];
+            if (scaled) vn = vn * vs;
+            v[c] = vn + (tk + td);
+        }
     }
 }
 
@@ -784,50 +851,166 @@ __global__ void k_scale_pending(long long len, const Scal *__restrict__ sc, doub
         u[i] = u[i] * ib;
 }
 
-// cblas_dnrm2 (mycblas.c:194-219) in its own sequential order, one lane.
-// Writes the norm to *out.  Exact-order mode only.
-__global__ void k_dnrm2_seq(int len, const double *__restrict__ v, double *out, const Scal *sc,
-                            int check_beta) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    if (sc && (sc->done || (check_beta && !sc->beta_pos))) return;
-    double scale = 0.0, ssq = 1.0;
-    if (len <= 0) {
-        *out = 0.0;
-        return;
-    }
-    if (len == 1) {
-        *out = fabs(v[0]);
-        return;
-    }
-    for (int i = 0; i < len; ++i) {
-        const double x = v[i];
-        if (x != 0.0) {
-            const double ax = fabs(x);
-            if (scale < ax) {
-                const double q = scale / ax;
-                ssq = 1.0 + ssq * q * q;
-                scale = ax;
-            } else {
-                const double q = ax / scale;
-                ssq += q * q;
-            }
+// Sequential sums in the reference's order (exact-order mode only).  Every
+// addition depends on the one before it, so one FP64 add latency per element
+// is the floor; the terms do not, so a workgroup of two wavefronts splits the
+// work: one forms the terms of the next SEQ_T elements with coalesced loads
+// (the divisions of dnrm2 64 at a time), the other adds the tile before it
+// from LDS.  One lane doing both took 55 ns per element (a division and a
+// load on the chain), this 3.8 (dknorm) to 4.6 (dnrm2): the three norms of an
+// iteration at 24^3 / 60k rays 335 us, 17.0 ms before.
+constexpr int SEQ_T = 512;
+
+// acc += term[0..N) in order, all lanes alike (broadcast LDS reads, the next
+// sixteen terms read ahead of the additions of the sixteen before them)
+template <int N>
+__device__ __forceinline__ double seq_add(double acc, const double *term) {
+    static_assert(N % 32 == 0, "two steps of sixteen terms");
+    const double2 *t2 = reinterpret_cast<const double2 *>(term);
+    double2 q[8], r[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[i] = t2[i];
+    for (int h = 0; h < N / 2; h += 16) {
+        const double2 *next = t2 + (h + 16 < N / 2 ? h + 16 : 0);  // the last step reads the first terms again
+#pragma unroll
+        for (int i = 0; i < 8; ++i) r[i] = t2[h + 8 + i];
+        __builtin_amdgcn_sched_barrier(0);  // the compiler would sink the reads to their uses
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            acc += q[i].x;
+            acc += q[i].y;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) q[i] = next[i];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            acc += r[i].x;
+            acc += r[i].y;
         }
     }
-    *out = scale * sqrt(ssq);
+    return acc;
 }
 
-// dknorm of lsqr.c:685-690 in the reference's order, one lane: reads the
-// w of before the update.  Exact-order mode only.
-__global__ void k_dknorm_seq(int n, const double *__restrict__ w, Scal *sc) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    if (sc->done) return;
-    const double t3 = sc->t3;
-    double dk = 0.0;
-    for (int i = 0; i < n; ++i) {
-        const double t = w[i];
-        dk = (t3 * t) * (t3 * t) + dk;
+struct SeqVec {
+    int len;
+    const double *v;
+    double *out;
+};
+
+// cblas_dnrm2 (mycblas.c:194-219) of the grid's vectors, workgroup b taking
+// vector b.  The reference keeps (scale, ssq): an element larger than the
+// scale so far gives ssq = 1 + ssq (scale/ax)^2 and becomes the scale, any
+// other nonzero one adds (ax/scale)^2.  The scale before an element is the
+// largest of the elements before it, a prefix maximum (NaN never compares
+// larger), so the terms can be formed ahead; term[i] holds the squared
+// quotient, or scale/ax where bit i of `big` marks a new scale.  Zeros add
+// nothing (+0 to an ssq >= 1).
+__global__ __launch_bounds__(128) void k_dnrm2_seq(SeqVec a, SeqVec b, const Scal *sc, int check_beta) {
+    __shared__ __align__(16) double term[2][SEQ_T];
+    __shared__ unsigned long long big[2][SEQ_T / kWave];
+    __shared__ double scale_end;
+    if (sc && (sc->done || (check_beta && !sc->beta_pos))) return;  // uniform
+    const SeqVec s = blockIdx.x == 0 ? a : b;
+    if (s.len <= 1) {
+        if (threadIdx.x == 0) *s.out = s.len <= 0 ? 0.0 : fabs(s.v[0]);
+        return;
     }
-    sc->dk_seq = dk;
+    constexpr int NG = SEQ_T / kWave;
+    const int lane = threadIdx.x % kWave;
+    const bool producer = threadIdx.x >= kWave;
+    const int tiles = (s.len + SEQ_T - 1) / SEQ_T;
+    double scale = 0.0, ssq = 1.0;
+    double x[NG];
+    auto load = [&](int t) {
+#pragma unroll
+        for (int g = 0; g < NG; ++g) {
+            x[g] = s.v[min((long long)t * SEQ_T + g * kWave + lane, (long long)s.len - 1)];
+        }
+    };
+    if (producer) load(0);
+    for (int t = 0; t <= tiles; ++t) {
+        if (producer && t < tiles) {
+#pragma unroll
+            for (int g = 0; g < NG; ++g) {
+                if ((long long)t * SEQ_T + g * kWave + lane >= s.len) x[g] = 0.0;
+                const double ax = fabs(x[g]);
+                double before = scale;
+                unsigned long long mask = 0;
+                if (__ballot(scale < ax) != 0) {
+                    double m = scale < ax ? ax : scale;
+#pragma unroll
+                    for (int o = 1; o < kWave; o <<= 1) {
+                        const double up = __shfl_up(m, o);
+                        if (lane >= o && m < up) m = up;
+                    }
+                    const double prev = __shfl_up(m, 1);
+                    if (lane > 0) before = prev;
+                    mask = __ballot(before < ax);
+                    scale = __shfl(m, kWave - 1);
+                }
+                const bool up = before < ax;
+                double q = (up ? before : ax) / (up ? ax : before);
+                if (!up) q = q * q;
+                term[t & 1][g * kWave + lane] = x[g] != 0.0 ? q : 0.0;
+                if (lane == 0) big[t & 1][g] = mask;
+            }
+            if (t + 1 < tiles) load(t + 1);
+            else if (lane == 0) scale_end = scale;
+        } else if (threadIdx.x == 0 && t > 0) {
+            const double *tt = term[(t - 1) & 1];
+            unsigned long long any = 0;
+#pragma unroll
+            for (int g = 0; g < NG; ++g) any |= big[(t - 1) & 1][g];
+            if (any == 0) ssq = seq_add<SEQ_T>(ssq, tt);
+            for (int g = 0; any != 0 && g < NG; ++g) {
+                const unsigned long long mask = big[(t - 1) & 1][g];
+                if (mask == 0) {
+                    ssq = seq_add<kWave>(ssq, tt + g * kWave);
+                } else {
+                    for (int i = 0; i < kWave; ++i) {
+                        const double q = tt[g * kWave + i];
+                        ssq = (mask >> i) & 1ull ? 1.0 + ssq * q * q : ssq + q;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *s.out = scale_end * sqrt(ssq);
+}
+
+// dknorm of lsqr.c:685-690 in the reference's order: reads the w of before
+// the update.
+__global__ __launch_bounds__(128) void k_dknorm_seq(int n, const double *__restrict__ w, Scal *sc) {
+    __shared__ __align__(16) double term[2][SEQ_T];
+    if (sc->done) return;  // uniform
+    const double t3 = sc->t3;
+    const int lane = threadIdx.x % kWave;
+    const bool producer = threadIdx.x >= kWave;
+    const int tiles = (n + SEQ_T - 1) / SEQ_T;
+    double dk = 0.0;
+    double x[SEQ_T / kWave];
+    auto load = [&](int t) {
+#pragma unroll
+        for (int g = 0; g < SEQ_T / kWave; ++g)
+            x[g] = w[min((long long)t * SEQ_T + g * kWave + lane, (long long)n - 1)];
+    };
+    if (producer) load(0);
+    for (int t = 0; t <= tiles; ++t) {
+        if (producer && t < tiles) {
+#pragma unroll
+            for (int g = 0; g < SEQ_T / kWave; ++g) {
+                const bool in = (long long)t * SEQ_T + g * kWave + lane < n;
+                term[t & 1][g * kWave + lane] = in ? (t3 * x[g]) * (t3 * x[g]) : 0.0;
+            }
+            if (t + 1 < tiles) load(t + 1);
+        } else if (threadIdx.x == 0 && t > 0) {
+            dk = seq_add<SEQ_T>(dk, term[(t - 1) & 1]);
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) sc->dk_seq = dk;
 }
 
 // ---------------------------------------------------------------------------
