@@ -7,21 +7,26 @@
 // channel 0 of a 32-channel tensor whose other channels are zero (input) or
 // ignored (output), so that every layer is the same 32 -> 32 convolution.
 //
-// A 3x3x3 convolution with zero padding is an implicit GEMM: M = voxels,
-// N = 32 output channels, K = 27 taps x 32 input channels.  One wavefront
-// owns 32 consecutive voxels x 32 output channels and issues 108
-// v_mfma_f32_32x32x8_bf16 (bf16 operands, FP32 accumulation):
-//   A (32 x 8):  lane l holds row l%32, k = 4*(l/32) .. +3
-//   B (8 x 32):  lane l holds column l%32, k = 4*(l/32) .. +3
+// A 3x3x3 convolution with zero padding is an implicit GEMM: M = 32 output
+// channels, N = voxels, K = 27 taps x 32 input channels, in steps of one
+// v_mfma_f32_32x32x16_bf16 (bf16 operands, FP32 accumulation):
+//   A (32 x 16): lane l holds row l%32, k = 8*(l/32) .. +7
+//   B (16 x 32): lane l holds column l%32, k = 8*(l/32) .. +7
 //   D (32 x 32): lane l, register r holds row 8*(r/4) + 4*(l/32) + r%4,
 //                column l%32
 // Weights are bf16 in [tap][out channel][in channel] order so that a lane's
-// four k values are contiguous.  Tap t = (dz+1)*9 + (dy+1)*3 + (dx+1) reads
+// eight k values are contiguous.  Tap t = (dz+1)*9 + (dy+1)*3 + (dx+1) reads
 // the neighbour at (x+dx, y+dy, z+dz); tap 26-t is its mirror.
+//
+// One 32x32x16 step adds its k = 0..7 and then its k = 8..15 exactly as two
+// 32x32x8 steps do (measured: no difference in 204,800 results over random
+// operands), at twice their rate, so results do not depend on which is used.
 #pragma once
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <type_traits>
 
 namespace plsqr {
 namespace cnn {
@@ -30,15 +35,13 @@ constexpr int C = 32;
 constexpr int TAPS = 27;
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t uint4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t uint2_t __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
-// float -> bf16 bits, round to nearest even (NaN stays NaN)
-__device__ __forceinline__ uint16_t f2bf(float f) {
-    uint32_t u = __float_as_uint(f);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
-}
+// float -> bf16 bits, round to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
@@ -56,61 +59,268 @@ __device__ __forceinline__ Vox vox_of(long long g, int nx, int ny, int V) {
     return r;
 }
 
+// two floats as packed bf16 bits, the first in the low half
+__device__ __forceinline__ uint32_t pack_bf(float lo, float hi) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, bf16x2{(__bf16)lo, (__bf16)hi});
+}
+
 // ---------------------------------------------------------------------------
 // out[g][n] = f(bias[n] + sum_t sum_k in[g + off(t)][k] * w[t][n][k]) for the
-// `total` (sample, voxel) rows; neighbours outside the grid read as zero.
-// f: ReLU when relu != 0; then, when mask is given, out = 0 where
+// (sample, voxel) rows g of `samples` grids; neighbours outside the grid read
+// as zero.  f: ReLU when relu != 0; then, when mask is given, out = 0 where
 // mask[g][n] <= 0 (the ReLU derivative of the layer below, for the data
-// gradient).  Writes bf16 (out_bf) and/or FP32 (out_f), each may be NULL.
-// Workgroups of 4 wavefronts; wavefront w of block b owns rows
-// [(4b + w) * 32, +32).
+// gradient; with OUT = CONV_BF16 only).
+//   IN   CONV_BF16 bf16 [g][32]; CONV_F32 FP32 [g][32], rounded to bf16 here;
+//        CONV_ONE FP32 [g], channel 0 of an input whose other channels are
+//        zero (their K steps, which would add zeros, are left out)
+//   WF32 the weights are FP32 (rounded here) instead of bf16
+//   OUT  CONV_BF16 bf16 [g][32] or CONV_F32 FP32 [g][32]
+//
+// A workgroup owns bricks of 8 x 8 x 8 voxels: the 10 x 10 x 10 neighbourhood
+// and all weights lie in LDS, so each input row is read from memory about
+// twice instead of 27 times and the 27 taps are LDS reads at constant offsets
+// from one address per lane.  Wavefront w computes plane w of the brick as two
+// 32-voxel columns (8 x 4) that share each weight fragment.  With only
+// the LDS reads and matrix steps left the kernel takes 59 us of the 87 below, the rate a large matrix product reaches
+// here.  A voxel takes 80 bytes of LDS for its 64 and a line of voxels 896, so
+// that the 16-byte reads of 16 lanes (8 in x, 2 in y) fall on different banks
+// (with lines of 800 bytes half of the LDS cycles were conflicts: 118 us).  One
+// workgroup per CU stays for all of its bricks (weights are staged
+// once); the next brick's rows are loaded into registers while this one is
+// summed.  Workgroup b takes bricks of the b % 8-th of eight contiguous ranges,
+// so neighbouring bricks share their halo in one XCD's L2.
+// 48^3, FP32 in and out: 16.2 us, 65 before (fragments loaded from
+// memory per tap: 56 us, and two passes that made bf16 copies); 67^3 x 4
+// samples, bf16: 87 us per layer, 478 before.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void kc_conv_fwd(int nx, int ny, int nz, long long total,
-                                                   const uint16_t *__restrict__ in, const uint16_t *__restrict__ w,
-                                                   const float *__restrict__ bias, const uint16_t *__restrict__ mask,
-                                                   int relu, uint16_t *__restrict__ out_bf, float *__restrict__ out_f) {
-    const int lane = threadIdx.x & 63;
-    const long long g0 = ((long long)blockIdx.x * 4 + threadIdx.x / 64) * 32;
-    if (g0 >= total) return;  // uniform per wavefront; no block barrier below
-    const int V = nx * ny * nz;
-    const int i = lane & 31, kq = lane >> 5;
-    const long long g = g0 + i;
-    const bool row_ok = g < total;
-    Vox p{0, 0, 0};
-    if (row_ok) p = vox_of(g, nx, ny, V);
-    floatx16 acc;
+enum { CONV_BF16 = 0, CONV_F32 = 1, CONV_ONE = 2 };
+constexpr int CB = 8;                    // brick edge
+constexpr int CH = CB + 2;               // with its halo
+constexpr int CONV_THREADS = 64 * CB;    // one wavefront per plane
+
+template <int IN, bool WF32, int OUT>
+__global__ __launch_bounds__(CONV_THREADS, 2) void kc_conv(int nx, int ny, int nz, int samples, const void *__restrict__ in,
+                                                           const void *__restrict__ w, const float *__restrict__ bias,
+                                                           const uint16_t *__restrict__ mask, int relu,
+                                                           void *__restrict__ out, int aligned) {
+    constexpr int KS = IN == CONV_ONE ? 1 : 2;       // K steps per tap
+    constexpr int VS = IN == CONV_ONE ? 3 : 5;       // 16-byte units per voxel in LDS (2 or 4 of data)
+    constexpr int CPV = IN == CONV_ONE ? 1 : 4;      // units loaded per voxel
+    constexpr int NV = CH * CH * CH;
+    // units per line and plane of the neighbourhood: a line is 8 (mod 16) units
+    // long, so the 16 lanes of a read cycle (8 in x, 2 in y) take 16 bank groups
+    constexpr int LP = IN == CONV_ONE ? 40 : 56, PP = CH * LP;
+    static_assert(LP >= CH * VS && LP % 16 == 8, "lines do not overlap and fall on different banks");
+    constexpr int PER = (NV * CPV + CONV_THREADS - 1) / CONV_THREADS;
+    __shared__ uint4_t wl[TAPS * KS * 64];
+    __shared__ uint4_t xl[CH * PP];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tx = (nx + CB - 1) / CB, ty = (ny + CB - 1) / CB, tz = (nz + CB - 1) / CB;
+    const int per_sample = tx * ty * tz, tiles = per_sample * samples;
+    // this workgroup's bricks: first, first + step, ... below last
+    const int queues = gridDim.x % 8 == 0 ? 8 : 1;
+    const int q = blockIdx.x % queues, step = gridDim.x / queues;
+    const int first = (int)((long long)tiles * q / queues) + blockIdx.x / queues;
+    const int last = (int)((long long)tiles * (q + 1) / queues);
+    if (first >= last) return;
+
+    // weight fragments, lane-linear: unit (t * KS + s) * 64 + l holds w[t][l%32][16 s + 8 (l/32) .. +7]
+    {
+        constexpr int NU = TAPS * KS * 64, WPER = (NU + CONV_THREADS - 1) / CONV_THREADS;
+        uint4_t u[WPER][WF32 ? 2 : 1];
+        const bool wide = ((uintptr_t)w & 15) == 0;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    for (int dz = -1; dz <= 1; ++dz)
-        for (int dy = -1; dy <= 1; ++dy) {
-            const bool yz_ok = row_ok && (unsigned)(p.z + dz) < (unsigned)nz && (unsigned)(p.y + dy) < (unsigned)ny;
+        for (int j = 0; j < WPER; ++j) {
+            const int i = min(tid + j * CONV_THREADS, NU - 1);
+            const int l = i & 63, s = (i >> 6) % KS, t = (i >> 6) / KS;
+            const int src = (t * C + (l & 31)) * C + 16 * s + 8 * (l >> 5);
+            if constexpr (!WF32) {
+                u[j][0] = *(const uint4_t *)((const uint16_t *)w + src);
+            } else if (wide) {
+                u[j][0] = ((const uint4_t *)((const float *)w + src))[0];
+                u[j][1] = ((const uint4_t *)((const float *)w + src))[1];
+            } else {
 #pragma unroll
-            for (int dx = -1; dx <= 1; ++dx) {
-                const int t = (dz + 1) * 9 + (dy + 1) * 3 + (dx + 1);
-                const bool ok = yz_ok && (unsigned)(p.x + dx) < (unsigned)nx;
-                const long long src = ok ? (g + (long long)dz * nx * ny + (long long)dy * nx + dx) * C : 0;
-                const uint16_t *wt = w + ((size_t)t * C + i) * C + kq * 4;
-                const uint16_t *at = in + src + kq * 4;
+                for (int k = 0; k < 8; ++k) u[j][k / 4][k % 4] = ((const uint32_t *)w)[src + k];
+            }
+        }
 #pragma unroll
-                for (int kc = 0; kc < 4; ++kc) {
-                    short4_t a = {0, 0, 0, 0};
-                    if (ok) a = *reinterpret_cast<const short4_t *>(at + kc * 8);
-                    const short4_t b = *reinterpret_cast<const short4_t *>(wt + kc * 8);
-                    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc, 0, 0, 0);
+        for (int j = 0; j < WPER; ++j) {
+            const int i = tid + j * CONV_THREADS;
+            if constexpr (WF32) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    u[j][0][k] = pack_bf(__uint_as_float(u[j][k / 2][2 * (k % 2)]), __uint_as_float(u[j][k / 2][2 * (k % 2) + 1]));
+            }
+            if (i < NU) wl[i] = u[j][0];
+        }
+    }
+    if constexpr (IN == CONV_ONE)  // channels 8..15 are zero
+        for (int p = tid; p < NV; p += CONV_THREADS)
+            xl[p / (CH * CH) * PP + p / CH % CH * LP + p % CH * VS + 1] = uint4_t{0, 0, 0, 0};
+
+    // the neighbourhood of a brick: loads into registers, then LDS
+    constexpr int RU = IN == CONV_F32 ? 2 : 1;
+    uint4_t reg[PER][RU];
+    // per unit, kept for all bricks: its voxel in the neighbourhood (bytes x, y,
+    // z) and its offset from the neighbourhood's first row, in units
+    int at[PER];
+    uint32_t off[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int i = tid + j * CONV_THREADS;
+        const int p = min(i / CPV, NV - 1), c = i % CPV;
+        const int px = p % CH, py = p / CH % CH, pz = p / (CH * CH);
+        at[j] = px | py << 8 | pz << 16;
+        off[j] = (uint32_t)((pz * ny + py) * nx + px) * CPV + c;
+    }
+    const uint32_t centre = (uint32_t)((ny + 1) * nx + 1) * CPV;  // a row of the brick itself
+    auto load = [&](int tile) {
+        const int sample = tile / per_sample, r = tile % per_sample;
+        const int x0 = (r % tx) * CB - 1, y0 = (r / tx % ty) * CB - 1, z0 = (r / (tx * ty)) * CB - 1;
+        const long long first_row = (((long long)sample * nz + z0) * ny + y0) * nx + x0;
+        constexpr int UB = IN == CONV_BF16 ? 16 : IN == CONV_F32 ? 32 : 4;  // bytes of a unit in memory
+        const uintptr_t from = (uintptr_t)in + first_row * (UB * CPV);
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const bool ok = (unsigned)(x0 + (at[j] & 255)) < (unsigned)nx && (unsigned)(y0 + (at[j] >> 8 & 255)) < (unsigned)ny &&
+                            (unsigned)(z0 + (at[j] >> 16)) < (unsigned)nz;
+            // outside: load a row of the brick and drop it (a predicated load would wait for itself)
+            const uintptr_t src = from + (uintptr_t)(ok ? off[j] : centre) * UB;
+            if constexpr (IN == CONV_BF16) {
+                reg[j][0] = *(const uint4_t *)src;
+                if (!ok) reg[j][0] = uint4_t{0, 0, 0, 0};
+            } else if constexpr (IN == CONV_F32) {
+                if (aligned) {
+                    reg[j][0] = ((const uint4_t *)src)[0];
+                    reg[j][1] = ((const uint4_t *)src)[1];
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) reg[j][k / 4][k % 4] = ((const uint32_t *)src)[k];
+                }
+                if (!ok) reg[j][0] = reg[j][1] = uint4_t{0, 0, 0, 0};
+            } else {
+                const uint32_t f = *(const uint32_t *)src;
+                reg[j][0][0] = ok ? f : 0u;
+            }
+        }
+    };
+    auto store = [&]() {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int i = tid + j * CONV_THREADS;
+            if (i >= NV * CPV) break;
+            const int to = (at[j] >> 16) * PP + (at[j] >> 8 & 255) * LP + (at[j] & 255) * VS + i % CPV;
+            uint4_t u = reg[j][0];
+            if constexpr (IN == CONV_F32) {
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    u[k] = pack_bf(__uint_as_float(reg[j][k / 2][2 * (k % 2)]), __uint_as_float(reg[j][k / 2][2 * (k % 2) + 1]));
+            } else if constexpr (IN == CONV_ONE) {
+                u = uint4_t{f2bf(__uint_as_float(reg[j][0][0])), 0, 0, 0};
+            }
+            xl[to] = u;
+        }
+    };
+
+    const int i = lane & 31, h = lane >> 5;
+    float bn[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bn[r] = bias ? bias[8 * (r / 4) + 4 * h + r % 4] : 0.f;
+    const uint4_t *xa = xl + wave * PP + (i >> 3) * LP + (i & 7) * VS + h;
+    load(first);
+    for (int tile = first; tile < last; tile += step) {
+        store();
+        __syncthreads();
+        if (tile + step < last) load(tile + step);
+        const int sample = tile / per_sample, rr = tile % per_sample;
+        const int x = (rr % tx) * CB + (i & 7), yb = (rr / tx % ty) * CB, z = (rr / (tx * ty)) * CB + wave;
+        if (z < nz) {  // uniform per wavefront
+            floatx16 acc[2];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[0][r] = acc[1][r] = 0.f;
+            const bool two = yb + 4 < ny;
+            // the mask rows are loaded before the sums: they would wait for
+            // memory after them (67^3 x 4: 119 -> 105 us per layer)
+            uint2_t mk[2][4];
+            if constexpr (OUT == CONV_BF16) {
+                if (mask) {
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        const long long g = (((long long)sample * nz + z) * ny + min(yb + 4 * e + (i >> 3), ny - 1)) * nx + min(x, nx - 1);
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) mk[e][b] = *(const uint2_t *)(mask + g * C + 8 * b + 4 * h);
+                    }
+                }
+            }
+            // groups of GS steps (fragments of one tap and K step): one group's
+            // fragments are read while the group before it is multiplied
+            auto sum = [&](auto halves) {
+                constexpr int NH = decltype(halves)::value, GS = 3, NG = TAPS * KS / GS;
+                static_assert(NG * GS == TAPS * KS, "whole groups");
+                bf16x8 a[2][GS], b[2][GS][NH];
+                auto read = [&](int gr) {
+#pragma unroll
+                    for (int k = 0; k < GS; ++k) {
+                        const int f = gr * GS + k, t = f / KS;
+                        a[gr & 1][k] = __builtin_bit_cast(bf16x8, wl[f * 64 + lane]);
+#pragma unroll
+                        for (int e = 0; e < NH; ++e)
+                            b[gr & 1][k][e] = __builtin_bit_cast(
+                                bf16x8, xa[t / 9 * PP + (t / 3 % 3 + 4 * e) * LP + t % 3 * VS + 2 * (f % KS)]);
+                    }
+                };
+                read(0);
+#pragma unroll
+                for (int gr = 0; gr < NG; ++gr) {
+                    if (gr + 1 < NG) read(gr + 1);
+                    __builtin_amdgcn_sched_barrier(0);  // the reads would sink to their uses
+#pragma unroll
+                    for (int k = 0; k < GS; ++k)
+#pragma unroll
+                        for (int e = 0; e < NH; ++e)
+                            acc[e] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[gr & 1][k], b[gr & 1][k][e], acc[e], 0, 0, 0);
+                }
+            };
+            if (two)
+                sum(std::integral_constant<int, 2>{});
+            else
+                sum(std::integral_constant<int, 1>{});
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int y = yb + 4 * e + (i >> 3);
+                if (x >= nx || y >= ny) continue;
+                const long long g = (((long long)sample * nz + z) * ny + y) * nx + x;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const long long o = g * C + 8 * b + 4 * h;  // channels 8b + 4h .. +3
+                    float v[4];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        v[k] = acc[e][4 * b + k] + bn[4 * b + k];
+                        if (relu) v[k] = fmaxf(v[k], 0.f);
+                    }
+                    if constexpr (OUT == CONV_BF16) {
+                        if (mask) {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k)
+                                if (!(bf2f((uint16_t)(mk[e][b][k / 2] >> (16 * (k % 2)))) > 0.f)) v[k] = 0.f;
+                        }
+                        *(uint2_t *)((uint16_t *)out + o) = uint2_t{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
+                    } else {
+                        float *d = (float *)out + o;
+                        if (aligned) {
+                            *(float4 *)d = make_float4(v[0], v[1], v[2], v[3]);
+                        } else {
+#pragma unroll
+                            for (int k = 0; k < 4; ++k) d[k] = v[k];
+                        }
+                    }
                 }
             }
         }
-    const int n = i;
-    const float bn = bias ? bias[n] : 0.f;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const long long gg = g0 + 8 * (r / 4) + 4 * kq + (r % 4);
-        if (gg >= total) continue;
-        float val = acc[r] + bn;
-        if (relu) val = fmaxf(val, 0.f);
-        if (mask && !(bf2f(mask[gg * C + n]) > 0.f)) val = 0.f;
-        if (out_bf) out_bf[gg * C + n] = f2bf(val);
-        if (out_f) out_f[gg * C + n] = val;
+        __syncthreads();
     }
 }
 

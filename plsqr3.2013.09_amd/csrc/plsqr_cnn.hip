@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -143,13 +144,31 @@ int prep_weights(plsqr_cnn *h) {
     return PLSQR_OK;
 }
 
-int conv_fwd(plsqr_cnn *h, long long total, const uint16_t *in, const uint16_t *w, const float *bias,
-             const uint16_t *mask, int relu, uint16_t *out_bf, float *out_f, hipStream_t st) {
-    const long long waves = (total + 31) / 32;
-    const long long blocks = (waves + 3) / 4;
-    hipLaunchKernelGGL(kc_conv_fwd, dim3((unsigned)blocks), dim3(256), 0, st, h ? h->nx : 0, h ? h->ny : 0,
-                       h ? h->nz : 0, total, in, w, bias, mask, relu, out_bf, out_f);
-    return PLSQR_OK;
+// Compute units of the current device, looked up once per device.
+int compute_units() {
+    constexpr int MAX_DEVICES = 64;
+    static std::atomic<int> known[MAX_DEVICES];
+    int dev = 0, cu = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) return 256;
+    if ((cu = known[dev].load(std::memory_order_relaxed)) > 0) return cu;
+    if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu < 1) cu = 256;
+    known[dev].store(cu, std::memory_order_relaxed);
+    return cu;
+}
+
+// One convolution layer over `samples` grids (kc_conv): one workgroup per CU,
+// or per brick where there are fewer; a multiple of eight when it can be, so
+// that each XCD takes one range of bricks.
+template <int IN, bool WF32, int OUT>
+void conv(int nx, int ny, int nz, int samples, const void *in, const void *w, const float *bias, const uint16_t *mask,
+          int relu, void *out, hipStream_t st) {
+    auto bricks = [](int n) { return (long long)((n + CB - 1) / CB); };
+    const long long tiles = bricks(nx) * bricks(ny) * bricks(nz) * samples;
+    long long g = std::min<long long>(tiles, compute_units());
+    if (g >= 8) g = g / 8 * 8;
+    const int aligned = (((uintptr_t)in | (uintptr_t)out) & 15) == 0;
+    hipLaunchKernelGGL((kc_conv<IN, WF32, OUT>), dim3((unsigned)g), dim3(CONV_THREADS), 0, st, nx, ny, nz, samples, in, w,
+                       bias, mask, relu, out, aligned);
 }
 
 // the network on h->xin (batch samples): activations act[0..3], zout
@@ -163,10 +182,15 @@ int forward(plsqr_cnn *h, int batch) {
     for (int l = 0; l < LAYERS; ++l) {
         const float *bias = h->params + (size_t)l * LSZ + WSZ;
         const bool last = l == LAYERS - 1;
-        const long long blocks = ((total + 31) / 32 + 3) / 4;
-        hipLaunchKernelGGL(kc_conv_fwd, dim3((unsigned)blocks), dim3(256), 0, h->stream, h->nx, h->ny, h->nz, total,
-                           h->act[l], h->wf[l], bias, (const uint16_t *)nullptr, last ? 0 : 1,
-                           last ? (uint16_t *)nullptr : h->act[l + 1], last ? h->zout : (float *)nullptr);
+        if (l == 0)
+            conv<CONV_ONE, false, CONV_BF16>(h->nx, h->ny, h->nz, batch, h->xin, h->wf[l], bias, nullptr, 1, h->act[1],
+                                             h->stream);
+        else if (!last)
+            conv<CONV_BF16, false, CONV_BF16>(h->nx, h->ny, h->nz, batch, h->act[l], h->wf[l], bias, nullptr, 1,
+                                              h->act[l + 1], h->stream);
+        else
+            conv<CONV_BF16, false, CONV_F32>(h->nx, h->ny, h->nz, batch, h->act[l], h->wf[l], bias, nullptr, 0, h->zout,
+                                             h->stream);
         CN_LAUNCH(h);
     }
     return PLSQR_OK;
@@ -211,10 +235,8 @@ int backward(plsqr_cnn *h, int batch) {
                         h->stream)))
             return rc;
         if (l > 0) {  // gradient of the layer's input, through the ReLU of layer l-1
-            const long long blocks = ((total + 31) / 32 + 3) / 4;
-            hipLaunchKernelGGL(kc_conv_fwd, dim3((unsigned)blocks), dim3(256), 0, h->stream, h->nx, h->ny, h->nz, total,
-                               h->dz[cur], h->wb[l], (const float *)nullptr, h->act[l], 0, h->dz[1 - cur],
-                               (float *)nullptr);
+            conv<CONV_BF16, false, CONV_BF16>(h->nx, h->ny, h->nz, batch, h->dz[cur], h->wb[l], nullptr, h->act[l], 0,
+                                              h->dz[1 - cur], h->stream);
             CN_LAUNCH(h);
             cur = 1 - cur;
         }
@@ -274,12 +296,14 @@ int load_samples(plsqr_cnn *h, int batch, const double *atb, const double *xs, s
 
 // ---------------------------------------------------------------------------
 // Allocation-free variant of plsqr_cnn_conv_forward for callers that cannot
-// allocate device memory (HIP graph capture, serving loops).  Its scratch --
-// the bf16 copy of the input and the two bf16 weight layouts -- lives in one
-// file-scope device array, fixed in size; each device holds its own copy,
-// found once per device with hipGetSymbolAddress.  Every element the kernels
-// read is written earlier in the same call, so no clearing is needed; calls
-// that overlap on one device share the array and race.
+// allocate device memory (HIP graph capture, serving loops): kc_conv rounds
+// the FP32 operands itself.  A call whose output overlaps its input or weights
+// needs copies of them first; that scratch -- the bf16 input and the two bf16
+// weight layouts -- lives in one file-scope device array, fixed in size; each
+// device holds its own copy, found once per device with hipGetSymbolAddress.
+// Every element the kernels read is written earlier in the same call, so no
+// clearing is needed; such calls that overlap on one device share the array
+// and race.
 // ---------------------------------------------------------------------------
 constexpr long long NOALLOC_MAX_ELEMS = 1LL << 22;  // batch * voxels * 32 channels of input
 constexpr size_t NOALLOC_BYTES = sizeof(uint16_t) * ((size_t)NOALLOC_MAX_ELEMS + 2 * (size_t)WSZ);
@@ -307,6 +331,11 @@ int scratch_ptr(void **out) {
     }
     *out = g_scratch_ptr[dev];
     return PLSQR_OK;
+}
+
+bool overlap(const void *a, size_t na, const void *b, size_t nb) {
+    const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+    return x < y + nb && y < x + na;
 }
 }  // namespace
 
@@ -542,20 +571,15 @@ int plsqr_cnn_conv_forward(int nx, int ny, int nz, int batch, const float *in, c
     if (nx < 1 || ny < 1 || nz < 1 || batch < 1 || !in || !w || !out) return set_err(nullptr, PLSQR_ERR_ARG, "bad arguments");
     const long long total = (long long)batch * nx * ny * nz;
     plsqr_cnn tmp;
-    tmp.nx = nx;
-    tmp.ny = ny;
-    tmp.nz = nz;
     plsqr_cnn *h = &tmp;
     float *din = nullptr, *dw = nullptr, *db = nullptr, *dout = nullptr;
-    uint16_t *bin = nullptr, *wf = nullptr, *wb = nullptr;
     int rc = PLSQR_OK;
     auto cleanup = [&]() {
         for (void *p : tmp.allocs) (void)hipFree(p);
         tmp.allocs.clear();
     };
     if ((rc = calloc_dev(h, &din, (size_t)total * C)) || (rc = calloc_dev(h, &dw, WSZ)) || (rc = calloc_dev(h, &db, C)) ||
-        (rc = calloc_dev(h, &dout, (size_t)total * C)) || (rc = calloc_dev(h, &bin, (size_t)total * C)) ||
-        (rc = calloc_dev(h, &wf, WSZ)) || (rc = calloc_dev(h, &wb, WSZ))) {
+        (rc = calloc_dev(h, &dout, (size_t)total * C))) {
         g_cnn_err = tmp.err;
         cleanup();
         return rc;
@@ -564,10 +588,7 @@ int plsqr_cnn_conv_forward(int nx, int ny, int nz, int batch, const float *in, c
     if (e == hipSuccess) e = hipMemcpy(dw, w, sizeof(float) * WSZ, hipMemcpyHostToDevice);
     if (e == hipSuccess && bias) e = hipMemcpy(db, bias, sizeof(float) * C, hipMemcpyHostToDevice);
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(kc_to_bf16, dim3(grid_for(total * C, 256, 4096)), dim3(256), 0, 0, total * C,
-                           (const float *)din, bin);
-        hipLaunchKernelGGL(kc_prep_weights, dim3((WSZ + 255) / 256), dim3(256), 0, 0, (const float *)dw, wf, wb);
-        conv_fwd(h, total, bin, wf, bias ? db : nullptr, nullptr, relu, nullptr, dout, 0);
+        conv<CONV_F32, true, CONV_F32>(nx, ny, nz, batch, din, dw, bias ? db : nullptr, nullptr, relu, dout, 0);
         e = hipGetLastError();
         if (e == hipSuccess) e = hipDeviceSynchronize();
         if (e == hipSuccess) e = hipMemcpy(out, dout, sizeof(float) * total * C, hipMemcpyDeviceToHost);
@@ -588,19 +609,20 @@ int plsqr_cnn_conv_forward_noalloc(int nx, int ny, int nz, int batch, const floa
         return set_err(nullptr, PLSQR_ERR_ARG,
                        "batch * nx * ny * nz = " + std::to_string(total) + " exceeds the allocation-free limit of " +
                            std::to_string(NOALLOC_MAX_ELEMS / C) + " voxels");
-    void *base = nullptr;
-    int rc = scratch_ptr(&base);
-    if (rc) return rc;
-    uint16_t *bin = (uint16_t *)base;
-    uint16_t *wf = bin + NOALLOC_MAX_ELEMS, *wb = wf + WSZ;
     const hipStream_t st = (hipStream_t)stream;
-    plsqr_cnn tmp;  // grid only: no buffers
-    tmp.nx = nx;
-    tmp.ny = ny;
-    tmp.nz = nz;
-    hipLaunchKernelGGL(kc_to_bf16, dim3(grid_for(total * C, 256, 4096)), dim3(256), 0, st, total * C, in_dev, bin);
-    hipLaunchKernelGGL(kc_prep_weights, dim3((WSZ + 255) / 256), dim3(256), 0, st, w_dev, wf, wb);
-    conv_fwd(&tmp, total, bin, wf, bias_dev, nullptr, relu, nullptr, out_dev, st);
+    const size_t out_bytes = sizeof(float) * (size_t)total * C;
+    if (!overlap(in_dev, out_bytes, out_dev, out_bytes) && !overlap(w_dev, sizeof(float) * WSZ, out_dev, out_bytes)) {
+        conv<CONV_F32, true, CONV_F32>(nx, ny, nz, batch, in_dev, w_dev, bias_dev, nullptr, relu, out_dev, st);
+    } else {  // in place: the operands are copied to the scratch first
+        void *base = nullptr;
+        int rc = scratch_ptr(&base);
+        if (rc) return rc;
+        uint16_t *bin = (uint16_t *)base;
+        uint16_t *wf = bin + NOALLOC_MAX_ELEMS, *wb = wf + WSZ;
+        hipLaunchKernelGGL(kc_to_bf16, dim3(grid_for(total * C, 256, 4096)), dim3(256), 0, st, total * C, in_dev, bin);
+        hipLaunchKernelGGL(kc_prep_weights, dim3((WSZ + 255) / 256), dim3(256), 0, st, w_dev, wf, wb);
+        conv<CONV_BF16, false, CONV_F32>(nx, ny, nz, batch, bin, wf, bias_dev, nullptr, relu, out_dev, st);
+    }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_err(nullptr, PLSQR_ERR_HIP, std::string("conv forward: ") + hipGetErrorString(e));
     return PLSQR_OK;
@@ -614,9 +636,6 @@ int plsqr_cnn_conv_backward(int nx, int ny, int nz, int batch, const float *in, 
         return set_err(nullptr, PLSQR_ERR_ARG, "bad arguments");
     const long long total = (long long)batch * nx * ny * nz;
     plsqr_cnn tmp;
-    tmp.nx = nx;
-    tmp.ny = ny;
-    tmp.nz = nz;
     plsqr_cnn *h = &tmp;
     const int nch = (int)((total + WCHUNK - 1) / WCHUNK), nb = (int)((total + BCHUNK - 1) / BCHUNK);
     float *fin = nullptr, *fw = nullptr, *fdo = nullptr, *fdi = nullptr, *gw = nullptr, *wpart = nullptr, *bpart = nullptr;
@@ -643,7 +662,7 @@ int plsqr_cnn_conv_backward(int nx, int ny, int nz, int batch, const float *in, 
         hipLaunchKernelGGL(kc_to_bf16, dim3(g), dim3(256), 0, 0, total * C, (const float *)fin, bin);
         hipLaunchKernelGGL(kc_to_bf16, dim3(g), dim3(256), 0, 0, total * C, (const float *)fdo, bdo);
         hipLaunchKernelGGL(kc_prep_weights, dim3((WSZ + 255) / 256), dim3(256), 0, 0, (const float *)fw, wf, wb);
-        conv_fwd(h, total, bdo, wb, nullptr, nullptr, 0, nullptr, fdi, 0);
+        conv<CONV_BF16, false, CONV_F32>(nx, ny, nz, batch, bdo, wb, nullptr, nullptr, 0, fdi, 0);
         rc = wgrad(h, nx, ny, nz, total, bin, bdo, gw, gw + WSZ, wpart, bpart, 0);
         e = hipGetLastError();
         if (e == hipSuccess) e = hipDeviceSynchronize();
