@@ -372,14 +372,193 @@ __global__ __launch_bounds__(256) void kc_conv_wgrad(int nx, int ny, int nz, lon
     for (int e = threadIdx.x; e < C * C; e += 256) dst[e] = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
 }
 
-// grad[t][e] = sum over chunks (in order) of part[t][chunk][e]
+// ---------------------------------------------------------------------------
+// The same partials bit for bit, for lines of at most a few hundred voxels.
+// TG taps per workgroup: 9 (one dz) or 3 (one dz and dy).  kc_conv_wgrad loads
+// both operands two bytes at a time from memory, computes every row's voxel
+// and runs the matrix cores at 2% (67^3 x 4 samples: 1783 us per layer); this
+// kernel takes 163.  Sub-blocks of `rows` rows of dout and the rows
+// of `in` that their taps read are staged in LDS, and ds_read_b64_tr_b16 gives
+// each lane four rows of its channel (the reduction dimension is rows, which
+// lie across the channels in memory).  A wavefront keeps the order of
+// kc_conv_wgrad's: it adds rows 8w .. 8w+7 of every 32, here two such steps
+// per 32x32x16 matrix step, and one dout fragment serves the TG taps.
+//
+// The rows of `in` are staged at padded positions: lines of nx + 2 and planes
+// of ny + 2 lines with zeros in the padding, shifted by dz, so a tap is one
+// offset for all rows and needs no test; tab[r] is the position that row r's
+// middle tap reads.
+// 79 KB of LDS, so two workgroups share a CU and one stages while the other
+// multiplies; workgroup b works in the b % 8-th of eight contiguous ranges of
+// chunks, so the tap groups of a chunk and its neighbours share an XCD's L2.
+// The host picks TG (few chunks: 3, three times as many workgroups) and rows
+// (the most that fit), and calls it only where rows and positions fit 31 bits.
+// ---------------------------------------------------------------------------
+constexpr int WGRAD_UNITS = 5056;  // 16-byte units of LDS
+
+template <int TG>
+__global__ __launch_bounds__(256, 2) void kc_wgrad(int nx, int ny, int nz, int total, int chunk_len, int rows,
+                                                   const uint16_t *__restrict__ in, const uint16_t *__restrict__ dout,
+                                                   float *__restrict__ part) {
+    static_assert(TG == 3 || TG == 9, "the taps of one (dz, dy) or of one dz");
+    constexpr int GROUPS = TAPS / TG;
+    __shared__ uint4_t buf[WGRAD_UNITS];
+    const int nch = (total + chunk_len - 1) / chunk_len, jobs = nch * GROUPS;
+    const int q = blockIdx.x % 8, job = (int)((long long)jobs * q / 8) + blockIdx.x / 8;
+    if (job >= (int)((long long)jobs * (q + 1) / 8)) return;
+    const int chunk = job / GROUPS, group = job % GROUPS;
+    const int dz = (TG == 9 ? group : group / 3) - 1;
+    const int W = nx + 2, H = ny + 2;
+    const int line = TG == 9 ? 0 : (group % 3 - 1) * W;  // the tap group's line
+    const int lead = (TG == 9 ? W : 0) + 1 - line, tail = (TG == 9 ? W : 0) + 1 + line;  // positions around the row
+    auto position = [&](int g) -> int {
+        const int l = g / nx, plane = l / ny;
+        return (plane * H + (l - plane * ny) + 1) * W + (g - l * nx) + 1;
+    };
+    uint4_t *da = buf, *xa = buf + rows * 4;
+    uint16_t *tab = (uint16_t *)(buf + WGRAD_UNITS) - rows;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int s16 = lane & 15, h = lane >> 5;
+    const int lrow = wave * 8 + 32 * h + (s16 >> 2);              // this lane's row of a step's first four
+    const int lbyte = ((lane >> 4) & 1) * 32 + (s16 & 3) * 8;     // its channels in the row
+    typedef __attribute__((address_space(3))) short4_t lds_short4;
+    typedef __attribute__((address_space(3))) char lds_char;
+    lds_char *const dl = (lds_char *)da + lbyte, *const xb = (lds_char *)xa + lbyte;
+    auto transposed = [](lds_char *p) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)p); };
+    floatx16 acc[TG];
+#pragma unroll
+    for (int t = 0; t < TG; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
+    const int c0 = chunk * chunk_len, c1 = min(c0 + chunk_len, total);
+    for (int s = c0; s < c1; s += rows) {
+        const int live = min(rows, c1 - s);
+        const int lo = position(s) - lead;
+        const int n = position(s + live - 1) + tail - lo + 1;
+        // dout, zero past the chunk; position n of `in` is the zero row
+#pragma unroll 1
+        for (int i = tid; i < rows * 4; i += 4 * 256) {
+            uint4_t u[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                u[k] = ((const uint4_t *)dout)[s * 4 + min(i + k * 256, live * 4 - 1)];
+                if (i + k * 256 >= live * 4) u[k] = uint4_t{0, 0, 0, 0};
+            }
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                if (i + k * 256 < rows * 4) da[i + k * 256] = u[k];
+        }
+        {
+            const int c = tid & 3;
+            const int first = lo + (tid >> 2), fl = first / W;
+            int px = first - fl * W, plane = fl / H, py = fl - plane * H, pz = plane % nz;
+            // a step of 64 positions
+            const int sx = 64 % W, sy = 64 / W % H, sz = 64 / (W * H);
+            const int planes = total / (nx * ny);
+#pragma unroll 1
+            for (int i = tid >> 2; i <= n;) {
+                uint4_t u[4];
+                const int i0 = i;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const bool ok = i < n && px >= 1 && px <= nx && py >= 1 && py <= ny && plane < planes &&
+                                    (unsigned)(pz + dz) < (unsigned)nz;
+                    const int row = ok ? ((plane + dz) * ny + py - 1) * nx + px - 1 : 0;
+                    u[k] = ((const uint4_t *)in)[row * 4 + c];
+                    if (!ok) u[k] = uint4_t{0, 0, 0, 0};
+                    i += 64;
+                    px += sx;
+                    py += sy;
+                    int up = sz;
+                    if (px >= W) {
+                        px -= W;
+                        ++py;
+                    }
+                    if (py >= H) {
+                        py -= H;
+                        ++up;
+                    }
+                    plane += up;
+                    pz += up;
+                    while (pz >= nz) pz -= nz;
+                }
+#pragma unroll
+                for (int k = 0; k < 4; ++k)
+                    if (i0 + 64 * k <= n) xa[(i0 + 64 * k) * 4 + c] = u[k];
+            }
+        }
+#pragma unroll 1
+        for (int r = tid; r < rows; r += 256) tab[r] = (uint16_t)(r < live ? position(s + r) - lo + line : n);
+        __syncthreads();
+#pragma unroll 1
+        for (int r0 = 0; r0 < live; r0 += 64) {
+            typedef short short8_t __attribute__((ext_vector_type(8)));
+            short4_t af[2];
+            lds_char *x[2];  // the line of taps (dz, -1 or this dy)
+            int one[2], ln[2];
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                const int r = r0 + lrow + 4 * p;
+                af[p] = transposed(dl + r * (C * 2));
+                // bytes to the next position and line; rows past the end read the zero row for every tap
+                one[p] = r < live ? C * 2 : 0;
+                ln[p] = W * one[p];
+                x[p] = xb + tab[r] * (C * 2) - (TG == 9 ? ln[p] : 0);
+            }
+            const bf16x8 a = __builtin_bit_cast(bf16x8, __builtin_shufflevector(af[0], af[1], 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+            for (int dy = 0; dy < TG / 3; ++dy) {
+                short4_t bf[3][2];
+#pragma unroll
+                for (int p = 0; p < 2; ++p) {
+                    if (dy > 0) x[p] += ln[p];
+                    bf[0][p] = transposed(x[p] - one[p]);
+                    bf[1][p] = transposed(x[p]);
+                    bf[2][p] = transposed(x[p] + one[p]);
+                }
+#pragma unroll
+                for (int dx = 0; dx < 3; ++dx) {
+                    const short8_t b = __builtin_shufflevector(bf[dx][0], bf[dx][1], 0, 1, 2, 3, 4, 5, 6, 7);
+                    acc[dy * 3 + dx] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, __builtin_bit_cast(bf16x8, b),
+                                                                               acc[dy * 3 + dx], 0, 0, 0);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    // the four wavefronts' sums in order
+    float *red = (float *)buf;
+    const int i = lane & 31;
+#pragma unroll
+    for (int t = 0; t < TG; ++t) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[wave * C * C + (8 * (r / 4) + 4 * h + r % 4) * C + i] = acc[t][r];
+        __syncthreads();
+        float *dst = part + ((size_t)(group * TG + t) * nch + chunk) * (C * C);
+        for (int e = tid; e < C * C; e += 256)
+            dst[e] = ((red[e] + red[C * C + e]) + red[2 * C * C + e]) + red[3 * C * C + e];
+        __syncthreads();
+    }
+}
+
+// grad[t][e] = sum over chunks (in order) of part[t][chunk][e]; sixteen loads
+// in flight per thread, so the serial sum waits for memory once in sixteen
+// chunks (67^3 x 4: 294 chunks, 71 -> 15 us)
 __global__ void kc_wgrad_reduce(int nchunk, const float *__restrict__ part, float *__restrict__ grad) {
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= TAPS * C * C) return;
     const int t = idx / (C * C), e = idx % (C * C);
     const float *p = part + (size_t)t * nchunk * (C * C) + e;
     float s = 0.f;
-    for (int c = 0; c < nchunk; ++c) s += p[(size_t)c * (C * C)];
+    int c = 0;
+    for (; c + 16 <= nchunk; c += 16) {
+        float v[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = p[(size_t)(c + k) * (C * C)];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) s += v[k];
+    }
+    for (; c < nchunk; ++c) s += p[(size_t)c * (C * C)];
     grad[idx] = s;
 }
 

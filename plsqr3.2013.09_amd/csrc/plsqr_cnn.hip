@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <climits>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -196,10 +197,36 @@ int forward(plsqr_cnn *h, int batch) {
     return PLSQR_OK;
 }
 
+// Rows per sub-block of kc_wgrad<tg>: the most (a multiple of 64, at most 512)
+// whose dout rows, staged positions and table fit its LDS for every start row;
+// 0 when not even 64 do (lines of several hundred voxels) or when indices
+// would not fit 31 bits.
+int wgrad_rows(int nx, int ny, long long total, int tg) {
+    const long long W = nx + 2, plane = (long long)nx * ny;
+    if (total > (1 << 28) || total / plane * (ny + 2) * W > INT_MAX) return 0;
+    for (int r = 512; r >= 64; r -= 64) {
+        const long long lines = (r + nx - 2) / nx, planes = (r + plane - 2) / plane;  // boundaries crossed at most
+        const long long span = r + 2 * lines + 2 * W * planes + (tg == 9 ? 2 * W : 0) + 2;
+        if (r * 4 + (span + 1) * 4 + r / 8 <= WGRAD_UNITS) return r;
+    }
+    return 0;
+}
+
 int wgrad(plsqr_cnn *h, int nx, int ny, int nz, long long total, const uint16_t *in, const uint16_t *dout, float *gw,
           float *gb, float *wpart, float *bpart, hipStream_t st) {
     const int nch = (int)((total + WCHUNK - 1) / WCHUNK);
-    hipLaunchKernelGGL(kc_conv_wgrad, dim3(nch, TAPS), dim3(256), 0, st, nx, ny, nz, total, WCHUNK, in, dout, wpart);
+    // nine taps per workgroup once that fills the chip's 512 slots, else three
+    const int tg = nch * 3 >= 512 && wgrad_rows(nx, ny, total, 9) > 0 ? 9 : 3;
+    const int rows = wgrad_rows(nx, ny, total, tg);
+    const unsigned blocks = (unsigned)((nch * (TAPS / tg) + 7) / 8 * 8);
+    if (rows == 0)
+        hipLaunchKernelGGL(kc_conv_wgrad, dim3(nch, TAPS), dim3(256), 0, st, nx, ny, nz, total, WCHUNK, in, dout, wpart);
+    else if (tg == 9)
+        hipLaunchKernelGGL((kc_wgrad<9>), dim3(blocks), dim3(256), 0, st, nx, ny, nz, (int)total, WCHUNK,
+                           rows, in, dout, wpart);
+    else
+        hipLaunchKernelGGL((kc_wgrad<3>), dim3(blocks), dim3(256), 0, st, nx, ny, nz, (int)total, WCHUNK,
+                           rows, in, dout, wpart);
     hipLaunchKernelGGL(kc_wgrad_reduce, dim3((WSZ + 255) / 256), dim3(256), 0, st, nch, (const float *)wpart, gw);
     const int nb = (int)((total + BCHUNK - 1) / BCHUNK);
     hipLaunchKernelGGL(kc_bgrad, dim3(nb), dim3(256), 0, st, total, BCHUNK, dout, bpart);
