@@ -6,6 +6,8 @@
 // (sample, voxel) index; the network's one input and one output channel are
 // channel 0 of a 32-channel tensor whose other channels are zero (input) or
 // ignored (output), so that every layer is the same 32 -> 32 convolution.
+// Those two tensors, and the gradient of the output, are stored as that one
+// channel (FP32 [g]); the kernels supply the zeros.
 //
 // A 3x3x3 convolution with zero padding is an implicit GEMM: M = 32 output
 // channels, N = voxels, K = 27 taps x 32 input channels, in steps of one
@@ -75,7 +77,8 @@ __device__ __forceinline__ uint32_t pack_bf(float lo, float hi) {
 //        CONV_ONE FP32 [g], channel 0 of an input whose other channels are
 //        zero (their K steps, which would add zeros, are left out)
 //   WF32 the weights are FP32 (rounded here) instead of bf16
-//   OUT  CONV_BF16 bf16 [g][32] or CONV_F32 FP32 [g][32]
+//   OUT  CONV_BF16 bf16 [g][32], CONV_F32 FP32 [g][32] or CONV_ONE FP32 [g]
+//        (channel 0)
 //
 // A workgroup owns bricks of 8 x 8 x 8 voxels: the 10 x 10 x 10 neighbourhood
 // and all weights lie in LDS, so each input row is read from memory about
@@ -308,6 +311,8 @@ __global__ __launch_bounds__(CONV_THREADS, 2) void kc_conv(int nx, int ny, int n
                                 if (!(bf2f((uint16_t)(mk[e][b][k / 2] >> (16 * (k % 2)))) > 0.f)) v[k] = 0.f;
                         }
                         *(uint2_t *)((uint16_t *)out + o) = uint2_t{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
+                    } else if constexpr (OUT == CONV_ONE) {
+                        if (b == 0 && h == 0) ((float *)out)[g] = v[0];
                     } else {
                         float *d = (float *)out + o;
                         if (aligned) {
@@ -324,197 +329,174 @@ __global__ __launch_bounds__(CONV_THREADS, 2) void kc_conv(int nx, int ny, int n
     }
 }
 
-// ---------------------------------------------------------------------------
-// Weight gradient: part[(t * gridDim.x + chunk)][n][k] = sum over the chunk's
-// rows g of dout[g][n] * in[g + off(t)][k] (neighbours outside the grid are
-// zero).  blockIdx.x = chunk of chunk_len rows, blockIdx.y = tap; the 4
-// wavefronts take 8-row steps (MFMA reduction dimension = rows) and their
-// 32 x 32 results are summed in wavefront order.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void kc_conv_wgrad(int nx, int ny, int nz, long long total, int chunk_len,
-                                                     const uint16_t *__restrict__ in,
-                                                     const uint16_t *__restrict__ dout, float *__restrict__ part) {
-    __shared__ float red[4][C * C];
-    const int t = blockIdx.y;
-    const int dz = t / 9 - 1, dy = (t / 3) % 3 - 1, dx = t % 3 - 1;
-    const long long off = (long long)dz * nx * ny + (long long)dy * nx + dx;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
-    const int i = lane & 31, kq = lane >> 5;
-    const int V = nx * ny * nz;
-    const long long c0 = (long long)blockIdx.x * chunk_len;
-    const long long c1 = c0 + chunk_len < total ? c0 + chunk_len : total;
-    floatx16 acc;
+// s + this thread's rows q, q + 8, .. of the first `live` rows of staged dout
+// (a multiple of 64 rows is readable), thread (q, n) = (tid / 32, tid % 32)
+__device__ __forceinline__ float bias_rows(float s, const uint16_t *rows, int live) {
+    for (int r = threadIdx.x / C; r < live; r += 64) {
+        float v[8];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    for (long long gs = c0 + wave * 8; gs < c1; gs += 32) {
-        short4_t a, b;
+        for (int k = 0; k < 8; ++k) v[k] = bf2f(rows[(r + 8 * k) * C + threadIdx.x % C]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const long long g = gs + kq * 4 + j;
-            short av = 0, bv = 0;
-            if (g < c1) {
-                av = (short)dout[g * C + i];
-                const Vox p = vox_of(g, nx, ny, V);
-                if ((unsigned)(p.x + dx) < (unsigned)nx && (unsigned)(p.y + dy) < (unsigned)ny &&
-                    (unsigned)(p.z + dz) < (unsigned)nz)
-                    bv = (short)in[(g + off) * C + i];
-            }
-            a[j] = av;
-            b[j] = bv;
-        }
-        acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, b, acc, 0, 0, 0);
+        for (int k = 0; k < 8; ++k)
+            if (r + 8 * k < live) s += v[k];
     }
-    // D[row n][column k]: column = lane%32, rows per register
-#pragma unroll
-    for (int r = 0; r < 16; ++r) red[wave][(8 * (r / 4) + 4 * kq + (r % 4)) * C + i] = acc[r];
+    return s;
+}
+
+// A chunk's bias gradient: thread (q, n) = (tid / 32, tid % 32) holds the sum s
+// of rows q, q + 8, ..; the eight are added in order.  red: 256 floats of LDS.
+__device__ __forceinline__ void bias_partial(float s, float *red, float *__restrict__ part) {
+    red[threadIdx.x] = s;
     __syncthreads();
-    float *dst = part + ((size_t)t * gridDim.x + blockIdx.x) * (C * C);
-    for (int e = threadIdx.x; e < C * C; e += 256) dst[e] = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
+    if (threadIdx.x < C) {
+        float r = 0.f;
+        for (int k = 0; k < 8; ++k) r += red[k * C + threadIdx.x];
+        part[threadIdx.x] = r;
+    }
 }
 
 // ---------------------------------------------------------------------------
-// The same partials bit for bit, for lines of at most a few hundred voxels.
-// TG taps per workgroup: 9 (one dz) or 3 (one dz and dy).  kc_conv_wgrad loads
-// both operands two bytes at a time from memory, computes every row's voxel
-// and runs the matrix cores at 2% (67^3 x 4 samples: 1783 us per layer); this
-// kernel takes 163.  Sub-blocks of `rows` rows of dout and the rows
-// of `in` that their taps read are staged in LDS, and ds_read_b64_tr_b16 gives
-// each lane four rows of its channel (the reduction dimension is rows, which
-// lie across the channels in memory).  A wavefront keeps the order of
-// kc_conv_wgrad's: it adds rows 8w .. 8w+7 of every 32, here two such steps
-// per 32x32x16 matrix step, and one dout fragment serves the TG taps.
+// Weight gradient: part[t * nch + chunk][n][k] = sum over the chunk's rows g of
+// dout[g][n] * in[g + off(t)][k] (neighbours outside the grid are zero), and the
+// bias gradient's partials bpart[chunk][n].  DONE: dout is one channel, FP32
+// [g].  A wavefront w adds rows 8w .. 8w+7 of every 32 (the matrix reduction
+// dimension is rows, two such steps per 32x32x16), and the four wavefronts'
+// sums are added in order.
 //
-// The rows of `in` are staged at padded positions: lines of nx + 2 and planes
-// of ny + 2 lines with zeros in the padding, shifted by dz, so a tap is one
-// offset for all rows and needs no test; tab[r] is the position that row r's
-// middle tap reads.
-// 79 KB of LDS, so two workgroups share a CU and one stages while the other
-// multiplies; workgroup b works in the b % 8-th of eight contiguous ranges of
-// chunks, so the tap groups of a chunk and its neighbours share an XCD's L2.
-// The host picks TG (few chunks: 3, three times as many workgroups) and rows
-// (the most that fit), and calls it only where rows and positions fit 31 bits.
+// TG taps per workgroup: 9 (one dz) or 3 (one dz and dy); one dout fragment
+// serves them all.  Sub-blocks of 256 rows of dout and the contiguous rows of
+// `in` that their taps read are staged in LDS (a thread's loads for the next
+// sub-block are in flight while this one is multiplied), and
+// ds_read_b64_tr_b16 gives each lane four rows of its channel, which lie
+// across the channels in memory.  A tap is one offset from the row; near[r]
+// says which of a row's neighbours exist, and a tap without one reads a row of
+// zeros.  (Staging zero-padded lines instead needs no test, but finding each
+// staged row's place took 112 of 200 vector instructions per 9 matrix steps,
+// 182 us; loading both operands two bytes at a time from memory, tap by tap,
+// took 1783 us.)
+// 67^3 x 4 samples: 136 us per layer.
+//
+// Workgroup b works in the b % 8-th of eight contiguous ranges of chunks, so
+// the tap groups of a chunk and its neighbours share an XCD's L2.  The host
+// takes nine taps when lines are short enough for LDS and there are chunks
+// enough to fill the chip.
 // ---------------------------------------------------------------------------
-constexpr int WGRAD_UNITS = 5056;  // 16-byte units of LDS
+constexpr int WGRAD_R = 256;       // rows of dout per sub-block
+constexpr int WGRAD_XROWS = 640;   // staged rows of `in`: WGRAD_R + 2 (nx + 1) with nine taps
+constexpr int WGRAD_NX9 = (WGRAD_XROWS - WGRAD_R - 2) / 2;
 
-template <int TG>
-__global__ __launch_bounds__(256, 2) void kc_wgrad(int nx, int ny, int nz, int total, int chunk_len, int rows,
-                                                   const uint16_t *__restrict__ in, const uint16_t *__restrict__ dout,
-                                                   float *__restrict__ part) {
+template <int TG, bool DONE>
+__global__ __launch_bounds__(256, 2) void kc_wgrad(int nx, int ny, int nz, long long total, int chunk_len,
+                                                   const uint16_t *__restrict__ in, const void *__restrict__ dout,
+                                                   float *__restrict__ part, float *__restrict__ bpart) {
     static_assert(TG == 3 || TG == 9, "the taps of one (dz, dy) or of one dz");
-    constexpr int GROUPS = TAPS / TG;
-    __shared__ uint4_t buf[WGRAD_UNITS];
-    const int nch = (total + chunk_len - 1) / chunk_len, jobs = nch * GROUPS;
+    constexpr int GROUPS = TAPS / TG, R = WGRAD_R;
+    constexpr int XROWS = TG == 9 ? WGRAD_XROWS : R + 64, PA = R * 4 / 256, PX = XROWS * 4 / 256;
+    // bits of near[]: x-1, x+1, y-1, y+1 exist; the row is in the chunk and z+dz in the grid
+    __shared__ uint4_t da[R * 4];
+    __shared__ uint4_t xa[(XROWS + 1) * 4];  // the last row: zeros
+    __shared__ uint8_t near[R];
+    static_assert(sizeof(da) >= 4 * C * C * sizeof(float), "the wavefronts' sums pass through da");
+    const int nch = (int)((total + chunk_len - 1) / chunk_len), jobs = nch * GROUPS;
     const int q = blockIdx.x % 8, job = (int)((long long)jobs * q / 8) + blockIdx.x / 8;
     if (job >= (int)((long long)jobs * (q + 1) / 8)) return;
     const int chunk = job / GROUPS, group = job % GROUPS;
-    const int dz = (TG == 9 ? group : group / 3) - 1;
-    const int W = nx + 2, H = ny + 2;
-    const int line = TG == 9 ? 0 : (group % 3 - 1) * W;  // the tap group's line
-    const int lead = (TG == 9 ? W : 0) + 1 - line, tail = (TG == 9 ? W : 0) + 1 + line;  // positions around the row
-    auto position = [&](int g) -> int {
-        const int l = g / nx, plane = l / ny;
-        return (plane * H + (l - plane * ny) + 1) * W + (g - l * nx) + 1;
-    };
-    uint4_t *da = buf, *xa = buf + rows * 4;
-    uint16_t *tab = (uint16_t *)(buf + WGRAD_UNITS) - rows;
+    const int dz = (TG == 9 ? group : group / 3) - 1, dline = TG == 9 ? 0 : group % 3 - 1;
+    const int halo = (TG == 9 ? nx : 0) + 1, xunits = (R + 2 * halo) * 4;
+    const long long shift = ((long long)dz * ny + dline) * nx;  // row of the group's middle tap
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int s16 = lane & 15, h = lane >> 5;
+    const int s16 = lane & 15, h = lane >> 5, i = lane & 31;
     const int lrow = wave * 8 + 32 * h + (s16 >> 2);              // this lane's row of a step's first four
     const int lbyte = ((lane >> 4) & 1) * 32 + (s16 & 3) * 8;     // its channels in the row
     typedef __attribute__((address_space(3))) short4_t lds_short4;
     typedef __attribute__((address_space(3))) char lds_char;
     lds_char *const dl = (lds_char *)da + lbyte, *const xb = (lds_char *)xa + lbyte;
+    lds_char *const zeros = xb + XROWS * (C * 2);
     auto transposed = [](lds_char *p) { return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)p); };
+    const long long c0 = (long long)chunk * chunk_len, c1 = min(c0 + chunk_len, total);
+    uint4_t ua[PA], ux[PX];
+    auto load = [&](long long s) {
+        const int live = (int)min((long long)R, c1 - s);
+#pragma unroll
+        for (int k = 0; k < PA; ++k) {
+            const int unit = min(tid + k * 256, live * 4 - 1);
+            if constexpr (DONE)
+                ua[k] = uint4_t{unit % 4 == 0 ? f2bf(((const float *)dout)[s + unit / 4]) : 0u, 0, 0, 0};
+            else
+                ua[k] = ((const uint4_t *)dout + s * 4)[unit];
+            if (tid + k * 256 >= live * 4) ua[k] = uint4_t{0, 0, 0, 0};
+        }
+        // rows s + shift - halo .., clamped to the tensor (rows outside it are never used)
+        const long long r0 = s + shift - halo;
+        const int lo = (int)max(-r0, 0LL) * 4, hi = (int)max(min(total - r0, (long long)XROWS), 1 - r0) * 4 - 1;
+        const uint4_t *from = (const uint4_t *)in + r0 * 4;
+#pragma unroll
+        for (int k = 0; k < PX; ++k)
+            if (k * 256 < xunits) ux[k] = from[min(max(tid + k * 256, lo), hi)];
+    };
     floatx16 acc[TG];
 #pragma unroll
     for (int t = 0; t < TG; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
-    const int c0 = chunk * chunk_len, c1 = min(c0 + chunk_len, total);
-    for (int s = c0; s < c1; s += rows) {
-        const int live = min(rows, c1 - s);
-        const int lo = position(s) - lead;
-        const int n = position(s + live - 1) + tail - lo + 1;
-        // dout, zero past the chunk; position n of `in` is the zero row
+    float bsum = 0.f;
+    // this thread's row: its voxel, advanced by R rows per sub-block
+    const long long l0 = (c0 + tid) / nx, p0 = l0 / ny;
+    int vx = (int)(c0 + tid - l0 * nx), vy = (int)(l0 - p0 * ny), vz = (int)(p0 % nz);
+    const int sx = R % nx, sy = R / nx % ny, sz = R / nx / ny % nz;
+    if (tid < 4) xa[XROWS * 4 + tid] = uint4_t{0, 0, 0, 0};
+    load(c0);
 #pragma unroll 1
-        for (int i = tid; i < rows * 4; i += 4 * 256) {
-            uint4_t u[4];
+    for (long long s = c0; s < c1; s += R) {
+        const int live = (int)min((long long)R, c1 - s);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                u[k] = ((const uint4_t *)dout)[s * 4 + min(i + k * 256, live * 4 - 1)];
-                if (i + k * 256 >= live * 4) u[k] = uint4_t{0, 0, 0, 0};
-            }
+        for (int k = 0; k < PA; ++k) da[tid + k * 256] = ua[k];
 #pragma unroll
-            for (int k = 0; k < 4; ++k)
-                if (i + k * 256 < rows * 4) da[i + k * 256] = u[k];
+        for (int k = 0; k < PX; ++k)
+            if (k * 256 < xunits) xa[tid + k * 256] = ux[k];
+        near[tid] = (uint8_t)((vx > 0 ? 1 : 0) | (vx < nx - 1 ? 2 : 0) | (vy > 0 ? 4 : 0) | (vy < ny - 1 ? 8 : 0) |
+                              (tid < live && (unsigned)(vz + dz) < (unsigned)nz ? 16 : 0));
+        vx += sx;
+        vy += sy;
+        vz += sz;
+        if (vx >= nx) {
+            vx -= nx;
+            ++vy;
         }
-        {
-            const int c = tid & 3;
-            const int first = lo + (tid >> 2), fl = first / W;
-            int px = first - fl * W, plane = fl / H, py = fl - plane * H, pz = plane % nz;
-            // a step of 64 positions
-            const int sx = 64 % W, sy = 64 / W % H, sz = 64 / (W * H);
-            const int planes = total / (nx * ny);
-#pragma unroll 1
-            for (int i = tid >> 2; i <= n;) {
-                uint4_t u[4];
-                const int i0 = i;
-#pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const bool ok = i < n && px >= 1 && px <= nx && py >= 1 && py <= ny && plane < planes &&
-                                    (unsigned)(pz + dz) < (unsigned)nz;
-                    const int row = ok ? ((plane + dz) * ny + py - 1) * nx + px - 1 : 0;
-                    u[k] = ((const uint4_t *)in)[row * 4 + c];
-                    if (!ok) u[k] = uint4_t{0, 0, 0, 0};
-                    i += 64;
-                    px += sx;
-                    py += sy;
-                    int up = sz;
-                    if (px >= W) {
-                        px -= W;
-                        ++py;
-                    }
-                    if (py >= H) {
-                        py -= H;
-                        ++up;
-                    }
-                    plane += up;
-                    pz += up;
-                    while (pz >= nz) pz -= nz;
-                }
-#pragma unroll
-                for (int k = 0; k < 4; ++k)
-                    if (i0 + 64 * k <= n) xa[(i0 + 64 * k) * 4 + c] = u[k];
-            }
+        if (vy >= ny) {
+            vy -= ny;
+            ++vz;
         }
-#pragma unroll 1
-        for (int r = tid; r < rows; r += 256) tab[r] = (uint16_t)(r < live ? position(s + r) - lo + line : n);
+        if (vz >= nz) vz -= nz;
         __syncthreads();
+        if (s + R < c1) load(s + R);
+        if (group == GROUPS / 2) bsum = bias_rows(bsum, (const uint16_t *)da, live);
 #pragma unroll 1
         for (int r0 = 0; r0 < live; r0 += 64) {
             typedef short short8_t __attribute__((ext_vector_type(8)));
             short4_t af[2];
-            lds_char *x[2];  // the line of taps (dz, -1 or this dy)
-            int one[2], ln[2];
+            lds_char *x[2];  // first staged row of the tap group's first line, (dy, -1)
+            int has[2];
 #pragma unroll
             for (int p = 0; p < 2; ++p) {
                 const int r = r0 + lrow + 4 * p;
                 af[p] = transposed(dl + r * (C * 2));
-                // bytes to the next position and line; rows past the end read the zero row for every tap
-                one[p] = r < live ? C * 2 : 0;
-                ln[p] = W * one[p];
-                x[p] = xb + tab[r] * (C * 2) - (TG == 9 ? ln[p] : 0);
+                has[p] = near[r];
+                x[p] = xb + r * (C * 2);
             }
             const bf16x8 a = __builtin_bit_cast(bf16x8, __builtin_shufflevector(af[0], af[1], 0, 1, 2, 3, 4, 5, 6, 7));
 #pragma unroll
             for (int dy = 0; dy < TG / 3; ++dy) {
+                const int ly = TG == 9 ? dy - 1 : dline, need = 16 | (ly < 0 ? 4 : ly > 0 ? 8 : 0);
                 short4_t bf[3][2];
 #pragma unroll
                 for (int p = 0; p < 2; ++p) {
-                    if (dy > 0) x[p] += ln[p];
-                    bf[0][p] = transposed(x[p] - one[p]);
-                    bf[1][p] = transposed(x[p]);
-                    bf[2][p] = transposed(x[p] + one[p]);
+                    // a tap whose neighbour does not exist reads the row of zeros
+                    const bool in_y = (has[p] & need) == need;
+                    bf[0][p] = transposed(in_y && (has[p] & 1) ? x[p] : zeros);
+                    bf[1][p] = transposed((in_y ? x[p] : zeros - C * 2) + C * 2);
+                    bf[2][p] = transposed((in_y && (has[p] & 2) ? x[p] : zeros - 2 * C * 2) + 2 * C * 2);
+                    x[p] += nx * (C * 2);
                 }
 #pragma unroll
                 for (int dx = 0; dx < 3; ++dx) {
@@ -526,9 +508,12 @@ __global__ __launch_bounds__(256, 2) void kc_wgrad(int nx, int ny, int nz, int t
         }
         __syncthreads();
     }
+    float *red = (float *)da;
+    if (group == GROUPS / 2) {
+        bias_partial(bsum, red, bpart + (size_t)chunk * C);
+        __syncthreads();
+    }
     // the four wavefronts' sums in order
-    float *red = (float *)buf;
-    const int i = lane & 31;
 #pragma unroll
     for (int t = 0; t < TG; ++t) {
 #pragma unroll
@@ -541,51 +526,156 @@ __global__ __launch_bounds__(256, 2) void kc_wgrad(int nx, int ny, int nz, int t
     }
 }
 
-// grad[t][e] = sum over chunks (in order) of part[t][chunk][e]; sixteen loads
-// in flight per thread, so the serial sum waits for memory once in sixteen
-// chunks (67^3 x 4: 294 chunks, 71 -> 15 us)
-__global__ void kc_wgrad_reduce(int nchunk, const float *__restrict__ part, float *__restrict__ grad) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= TAPS * C * C) return;
-    const int t = idx / (C * C), e = idx % (C * C);
-    const float *p = part + (size_t)t * nchunk * (C * C) + e;
+// p[0] + p[stride] + .. (count terms, in order), sixteen loads in flight
+__device__ __forceinline__ float ordered_sum(const float *__restrict__ p, int count, size_t stride) {
     float s = 0.f;
     int c = 0;
-    for (; c + 16 <= nchunk; c += 16) {
+    for (; c + 16 <= count; c += 16) {
         float v[16];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = p[(size_t)(c + k) * (C * C)];
+        for (int k = 0; k < 16; ++k) v[k] = p[(size_t)(c + k) * stride];
 #pragma unroll
         for (int k = 0; k < 16; ++k) s += v[k];
     }
-    for (; c < nchunk; ++c) s += p[(size_t)c * (C * C)];
-    grad[idx] = s;
+    for (; c < count; ++c) s += p[(size_t)c * stride];
+    return s;
 }
 
-// bias gradient partials: part[block][n] = sum over the block's rows of dout[g][n]
-__global__ __launch_bounds__(256) void kc_bgrad(long long total, int chunk_len, const uint16_t *__restrict__ dout,
-                                                float *__restrict__ part) {
-    __shared__ float red[8][C];
-    const int n = threadIdx.x % C, q = threadIdx.x / C;
-    const long long c0 = (long long)blockIdx.x * chunk_len;
-    const long long c1 = c0 + chunk_len < total ? c0 + chunk_len : total;
-    float s = 0.f;
-    for (long long g = c0 + q; g < c1; g += 8) s += bf2f(dout[g * C + n]);
-    red[q][n] = s;
-    __syncthreads();
-    if (threadIdx.x < C) {
-        float r = 0.f;
-        for (int k = 0; k < 8; ++k) r += red[k][threadIdx.x];
-        part[(size_t)blockIdx.x * C + threadIdx.x] = r;
+// Sums over chunks in order.  Weights: grad[t][n][k] of part[t][chunk][n][k],
+// or with FIRST the one channel's grad[t][n][0] of part[chunk][n][t].  Bias
+// (the last workgroup): bgrad[n] of bpart[chunk][n].  The loads of sixteen
+// chunks are in flight together, so the serial sums wait for memory once in
+// sixteen (67^3 x 4: 294 chunks, weights 71 -> 15 us, bias 67 us before).
+template <bool FIRST>
+__global__ __launch_bounds__(256) void kc_grad_reduce(int nchunk, const float *__restrict__ part,
+                                                      const float *__restrict__ bpart, float *__restrict__ grad,
+                                                      float *__restrict__ bgrad) {
+    const int idx = blockIdx.x * 256 + threadIdx.x;
+    if (blockIdx.x == gridDim.x - 1) {
+        if (threadIdx.x < C) bgrad[threadIdx.x] = ordered_sum(bpart + threadIdx.x, nchunk, C);
+    } else if constexpr (FIRST) {
+        const int n = idx / C, t = idx % C;
+        if (n < C && t < TAPS) grad[(t * C + n) * C] = ordered_sum(part + idx, nchunk, C * C);
+    } else {
+        const int t = idx / (C * C), e = idx % (C * C);
+        if (t < TAPS) grad[idx] = ordered_sum(part + (size_t)t * nchunk * (C * C) + e, nchunk, C * C);
     }
 }
 
-__global__ void kc_bgrad_reduce(int nblk, const float *__restrict__ part, float *__restrict__ grad) {
-    const int n = threadIdx.x;
-    if (n >= C) return;
-    float s = 0.f;
-    for (int b = 0; b < nblk; ++b) s += part[(size_t)b * C + n];
-    grad[n] = s;
+// ---------------------------------------------------------------------------
+// Weight gradient of the first layer, whose input has one channel (FP32 [g]):
+// the 27 taps of that channel are the columns of one 32 x 32 product (the
+// other 31 channels' gradients are zero), so a chunk needs one matrix step
+// per 16 rows instead of 27 and no 32-channel copy of the input.  Rows are
+// added in kc_wgrad's order; part[chunk][n][t], and the bias partials.
+// Per sub-block of 256 rows: dout, read transposed; for each (dz, dy) the 258
+// inputs its three taps read; and one byte per row that says which neighbours
+// exist.  Lane (tap t) gathers its eight rows' inputs from LDS; the next
+// sub-block's loads are in flight meanwhile.  67^3 x 4 samples: 44 us
+// (kc_wgrad on a 32-channel copy: 136, and 41 for the copy).
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void kc_wgrad_first(int nx, int ny, int nz, long long total, int chunk_len,
+                                                      const float *__restrict__ x, const uint16_t *__restrict__ dout,
+                                                      float *__restrict__ part, float *__restrict__ bpart) {
+    constexpr int R = 256, WIN = R + 4;
+    __shared__ uint4_t da[R * 4];
+    __shared__ float win[9][WIN];
+    __shared__ __align__(8) uint8_t near[R];
+    static_assert(sizeof(da) >= 4 * C * C * sizeof(float), "the wavefronts' sums pass through da");
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int i = lane & 31, h = lane >> 5, s16 = lane & 15;
+    const int dz = i / 9 - 1, dy = i / 3 % 3 - 1, dx = i % 3 - 1;  // columns 27..31: no tap
+    // bits of near[]: the row is in the chunk; its neighbours at x-1, x+1, y-1, y+1, z-1, z+1 exist
+    const unsigned need = (i < TAPS ? 1u : 128u) | (dx < 0 ? 2u : dx > 0 ? 4u : 0u) | (dy < 0 ? 8u : dy > 0 ? 16u : 0u) |
+                          (dz < 0 ? 32u : dz > 0 ? 64u : 0u);
+    const float *xw = &win[i < TAPS ? i / 3 : 0][1 + dx];
+    typedef __attribute__((address_space(3))) short4_t lds_short4;
+    typedef __attribute__((address_space(3))) char lds_char;
+    lds_char *const dl = (lds_char *)da + ((lane >> 4) & 1) * 32 + (s16 & 3) * 8;
+    const int lrow = wave * 8 + 32 * h;
+    const long long c0 = (long long)blockIdx.x * chunk_len, c1 = min(c0 + chunk_len, total);
+    uint4_t ua[R * 4 / 256];
+    float uw[9], uedge = 0.f;  // windows' element tid, and the two past R of window tid / 2
+    auto load = [&](long long s) {
+        const int live = (int)min((long long)R, c1 - s);
+#pragma unroll
+        for (int k = 0; k < R * 4 / 256; ++k) {
+            ua[k] = ((const uint4_t *)(dout + s * C))[min(tid + k * 256, live * 4 - 1)];
+            if (tid + k * 256 >= live * 4) ua[k] = uint4_t{0, 0, 0, 0};
+        }
+        // element j of window (dz, dy) is row s + (dz ny + dy) nx - 1 + j; rows outside are never used
+        auto at = [&](int w, int j) {
+            const long long g = s + ((long long)(w / 3 - 1) * ny + (w % 3 - 1)) * nx - 1 + j;
+            return x[min(max(g, 0LL), total - 1)];
+        };
+#pragma unroll
+        for (int w = 0; w < 9; ++w) uw[w] = at(w, tid);
+        if (tid < 18) uedge = at(tid / 2, R + tid % 2);
+    };
+    floatx16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    float bsum = 0.f;
+    load(c0);
+    // this thread's row: its voxel, advanced by R rows per sub-block
+    const long long l0 = (c0 + tid) / nx, p0 = l0 / ny;
+    int vx = (int)(c0 + tid - l0 * nx), vy = (int)(l0 - p0 * ny), vz = (int)(p0 % nz);
+    const int sx = R % nx, sy = R / nx % ny, sz = (int)((long long)R / nx / ny % nz);
+#pragma unroll 1
+    for (long long s = c0; s < c1; s += R) {
+        const int live = (int)min((long long)R, c1 - s);
+#pragma unroll
+        for (int k = 0; k < R * 4 / 256; ++k) da[tid + k * 256] = ua[k];
+#pragma unroll
+        for (int w = 0; w < 9; ++w) win[w][tid] = uw[w];
+        if (tid < 18) win[tid / 2][R + tid % 2] = uedge;
+        near[tid] = (uint8_t)((tid < live ? 1 : 0) | (vx > 0 ? 2 : 0) | (vx < nx - 1 ? 4 : 0) | (vy > 0 ? 8 : 0) |
+                              (vy < ny - 1 ? 16 : 0) | (vz > 0 ? 32 : 0) | (vz < nz - 1 ? 64 : 0));
+        vx += sx;
+        vy += sy;
+        vz += sz;
+        if (vx >= nx) {
+            vx -= nx;
+            ++vy;
+        }
+        if (vy >= ny) {
+            vy -= ny;
+            ++vz;
+        }
+        if (vz >= nz) vz -= nz;
+        __syncthreads();
+        if (s + R < c1) load(s + R);
+        bsum = bias_rows(bsum, (const uint16_t *)da, live);
+#pragma unroll
+        for (int st = 0; st < R / 64; ++st) {
+            typedef short short8_t __attribute__((ext_vector_type(8)));
+            const int r0 = 64 * st + lrow;
+            short4_t af[2];
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                af[p] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4 *)(dl + (r0 + (s16 >> 2) + 4 * p) * (C * 2)));
+            const uint2_t f = *(const uint2_t *)(near + r0);
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                v[j] = xw[r0 + j];
+                if (((f[j / 4] >> (8 * (j % 4))) & need) != need) v[j] = 0.f;
+            }
+            const uint4_t b{pack_bf(v[0], v[1]), pack_bf(v[2], v[3]), pack_bf(v[4], v[5]), pack_bf(v[6], v[7])};
+            const short8_t a = __builtin_shufflevector(af[0], af[1], 0, 1, 2, 3, 4, 5, 6, 7);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+        }
+        __syncthreads();
+    }
+    float *red = (float *)da;
+    bias_partial(bsum, red, bpart + (size_t)blockIdx.x * C);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 16; ++r) red[wave * C * C + (8 * (r / 4) + 4 * h + r % 4) * C + i] = acc[r];
+    __syncthreads();
+    float *dst = part + (size_t)blockIdx.x * (C * C);
+    for (int e = tid; e < C * C; e += 256)
+        dst[e] = ((red[e] + red[C * C + e]) + red[2 * C * C + e]) + red[3 * C * C + e];
 }
 
 // bf16 weights of one layer: forward order wf[t][n][k] = W[t][n][k] and the
@@ -599,16 +689,6 @@ __global__ void kc_prep_weights(const float *__restrict__ W, uint16_t *__restric
     wb[((size_t)(TAPS - 1 - t) * C + k) * C + n] = h;
 }
 
-// a0[g][c] = bf16(x[g]) for c = 0, 0 otherwise (x: one value per row)
-__global__ void kc_expand_input(long long total, const float *__restrict__ x, uint16_t *__restrict__ a0) {
-    for (long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x; g < total; g += (long long)gridDim.x * blockDim.x) {
-        const uint16_t h = f2bf(x[g]);
-        uint16_t *row = a0 + g * C;
-        row[0] = h;
-        for (int c = 1; c < C; ++c) row[c] = 0;
-    }
-}
-
 // round an FP32 tensor to bf16
 __global__ void kc_to_bf16(long long len, const float *__restrict__ a, uint16_t *__restrict__ b) {
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < len; i += (long long)gridDim.x * blockDim.x)
@@ -616,26 +696,24 @@ __global__ void kc_to_bf16(long long len, const float *__restrict__ a, uint16_t 
 }
 
 // ---------------------------------------------------------------------------
-// Loss and its gradient.  Sample s of the batch has prediction z[g][0]
-// (g in its V rows) and target tgt[s*V + v] with tn[s] = ||tgt_s||^2:
+// Loss and its gradient.  Sample s of the batch has prediction z[g] (g in its
+// V rows) and target tgt[s*V + v] with tn[s] = ||tgt_s||^2:
 //   loss = (1/B) sum_s ||z_s - tgt_s||^2 / tn[s]
-//   dz[g][0] = bf16(2 (z - tgt) / (B tn[s])), other channels 0.
+//   dz[g] = 2 (z - tgt) / (B tn[s]), rounded to bf16.
 // part[s * nblk + block] = the block's share of ||z_s - tgt_s||^2.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void kc_loss(int V, int B, int nblk, const float *__restrict__ z,
                                                const float *__restrict__ tgt, const float *__restrict__ tn,
-                                               uint16_t *__restrict__ dz, float *__restrict__ part) {
+                                               float *__restrict__ dz, float *__restrict__ part) {
     __shared__ float red[256];
     const int s = blockIdx.y;
     float acc = 0.f;
     const float scale = 2.f / ((float)B * tn[s]);
     for (int v = blockIdx.x * 256 + threadIdx.x; v < V; v += nblk * 256) {
         const long long g = (long long)s * V + v;
-        const float d = z[g * C] - tgt[g];
+        const float d = z[g] - tgt[g];
         acc += d * d;
-        uint16_t *row = dz + g * C;
-        row[0] = f2bf(scale * d);
-        for (int c = 1; c < C; ++c) row[c] = 0;
+        dz[g] = bf2f(f2bf(scale * d));
     }
     red[threadIdx.x] = acc;
     __syncthreads();

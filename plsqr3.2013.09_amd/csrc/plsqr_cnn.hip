@@ -6,7 +6,6 @@
 
 #include <algorithm>
 #include <atomic>
-#include <climits>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -26,8 +25,7 @@ constexpr int WSZ = TAPS * C * C;      // weights of one layer
 constexpr int LSZ = WSZ + C;           // weights + bias
 constexpr int NPARAM = LAYERS * LSZ + 1;  // + the output gain (last entry, not trained)
 constexpr int GAIN = NPARAM - 1;
-constexpr int WCHUNK = 4096;           // rows per weight-gradient workgroup
-constexpr int BCHUNK = 4096;           // rows per bias-gradient workgroup
+constexpr int WCHUNK = 4096;           // rows per partial weight and bias gradient
 constexpr int LOSS_BLK = 64;           // workgroups per sample in the loss
 
 thread_local std::string g_cnn_err;
@@ -41,9 +39,9 @@ struct plsqr_cnn {
     uint8_t *mask = nullptr;
     uint16_t *wf[LAYERS] = {}, *wb[LAYERS] = {};
     bool weights_dirty = true;
-    uint16_t *act[LAYERS] = {};
-    float *zout = nullptr;
-    uint16_t *dz[2] = {};
+    uint16_t *act[LAYERS] = {};       // inputs of layers 1..3 (bf16, 32 channels; layer 0 reads xin)
+    float *zout = nullptr, *dz1 = nullptr;  // output and its gradient, one channel
+    uint16_t *dz[2] = {};             // gradients of the layers' outputs below
     float *wpart = nullptr, *bpart = nullptr, *lpart = nullptr;
     float *xin = nullptr, *tgt = nullptr, *tn = nullptr, *x0 = nullptr;
     int count = 0;
@@ -176,10 +174,6 @@ void conv(int nx, int ny, int nz, int samples, const void *in, const void *w, co
 int forward(plsqr_cnn *h, int batch) {
     int rc;
     if ((rc = prep_weights(h))) return rc;
-    const long long total = (long long)batch * h->V;
-    hipLaunchKernelGGL(kc_expand_input, dim3(grid_for(total, 256, 4096)), dim3(256), 0, h->stream, total, h->xin,
-                       h->act[0]);
-    CN_LAUNCH(h);
     for (int l = 0; l < LAYERS; ++l) {
         const float *bias = h->params + (size_t)l * LSZ + WSZ;
         const bool last = l == LAYERS - 1;
@@ -190,54 +184,48 @@ int forward(plsqr_cnn *h, int batch) {
             conv<CONV_BF16, false, CONV_BF16>(h->nx, h->ny, h->nz, batch, h->act[l], h->wf[l], bias, nullptr, 1,
                                               h->act[l + 1], h->stream);
         else
-            conv<CONV_BF16, false, CONV_F32>(h->nx, h->ny, h->nz, batch, h->act[l], h->wf[l], bias, nullptr, 0, h->zout,
+            conv<CONV_BF16, false, CONV_ONE>(h->nx, h->ny, h->nz, batch, h->act[l], h->wf[l], bias, nullptr, 0, h->zout,
                                              h->stream);
         CN_LAUNCH(h);
     }
     return PLSQR_OK;
 }
 
-// Rows per sub-block of kc_wgrad<tg>: the most (a multiple of 64, at most 512)
-// whose dout rows, staged positions and table fit its LDS for every start row;
-// 0 when not even 64 do (lines of several hundred voxels) or when indices
-// would not fit 31 bits.
-int wgrad_rows(int nx, int ny, long long total, int tg) {
-    const long long W = nx + 2, plane = (long long)nx * ny;
-    if (total > (1 << 28) || total / plane * (ny + 2) * W > INT_MAX) return 0;
-    for (int r = 512; r >= 64; r -= 64) {
-        const long long lines = (r + nx - 2) / nx, planes = (r + plane - 2) / plane;  // boundaries crossed at most
-        const long long span = r + 2 * lines + 2 * W * planes + (tg == 9 ? 2 * W : 0) + 2;
-        if (r * 4 + (span + 1) * 4 + r / 8 <= WGRAD_UNITS) return r;
-    }
-    return 0;
-}
-
-int wgrad(plsqr_cnn *h, int nx, int ny, int nz, long long total, const uint16_t *in, const uint16_t *dout, float *gw,
+// Weight and bias gradients of one layer; DONE: dout is one channel (FP32).
+template <bool DONE>
+int wgrad(plsqr_cnn *h, int nx, int ny, int nz, long long total, const uint16_t *in, const void *dout, float *gw,
           float *gb, float *wpart, float *bpart, hipStream_t st) {
     const int nch = (int)((total + WCHUNK - 1) / WCHUNK);
-    // nine taps per workgroup once that fills the chip's 512 slots, else three
-    const int tg = nch * 3 >= 512 && wgrad_rows(nx, ny, total, 9) > 0 ? 9 : 3;
-    const int rows = wgrad_rows(nx, ny, total, tg);
-    const unsigned blocks = (unsigned)((nch * (TAPS / tg) + 7) / 8 * 8);
-    if (rows == 0)
-        hipLaunchKernelGGL(kc_conv_wgrad, dim3(nch, TAPS), dim3(256), 0, st, nx, ny, nz, total, WCHUNK, in, dout, wpart);
-    else if (tg == 9)
-        hipLaunchKernelGGL((kc_wgrad<9>), dim3(blocks), dim3(256), 0, st, nx, ny, nz, (int)total, WCHUNK,
-                           rows, in, dout, wpart);
+    // nine taps per workgroup where a line fits and they fill the chip's 512
+    // slots (two workgroups per CU), else three: three times as many workgroups
+    const bool nine = nx <= WGRAD_NX9 && nch * 3 >= 512;
+    const unsigned blocks = (unsigned)((nch * (nine ? 3 : 9) + 7) / 8 * 8);
+    if (nine)
+        hipLaunchKernelGGL((kc_wgrad<9, DONE>), dim3(blocks), dim3(256), 0, st, nx, ny, nz, total, WCHUNK, in, dout, wpart,
+                           bpart);
     else
-        hipLaunchKernelGGL((kc_wgrad<3>), dim3(blocks), dim3(256), 0, st, nx, ny, nz, (int)total, WCHUNK,
-                           rows, in, dout, wpart);
-    hipLaunchKernelGGL(kc_wgrad_reduce, dim3((WSZ + 255) / 256), dim3(256), 0, st, nch, (const float *)wpart, gw);
-    const int nb = (int)((total + BCHUNK - 1) / BCHUNK);
-    hipLaunchKernelGGL(kc_bgrad, dim3(nb), dim3(256), 0, st, total, BCHUNK, dout, bpart);
-    hipLaunchKernelGGL(kc_bgrad_reduce, dim3(1), dim3(C), 0, st, nb, (const float *)bpart, gb);
+        hipLaunchKernelGGL((kc_wgrad<3, DONE>), dim3(blocks), dim3(256), 0, st, nx, ny, nz, total, WCHUNK, in, dout, wpart,
+                           bpart);
+    hipLaunchKernelGGL((kc_grad_reduce<false>), dim3(WSZ / 256 + 1), dim3(256), 0, st, nch, (const float *)wpart,
+                       (const float *)bpart, gw, gb);
     return hipGetLastError() == hipSuccess ? PLSQR_OK : set_err(h, PLSQR_ERR_HIP, "gradient kernels failed to launch");
 }
 
-// loss of zout against tgt/tn (batch samples), dz[0] = its gradient; *loss on the host
+// The first layer's; its gradients of the padded input channels stay zero.
+int wgrad_first(plsqr_cnn *h, long long total, const uint16_t *dout, float *gw, float *gb) {
+    const int nch = (int)((total + WCHUNK - 1) / WCHUNK);
+    hipLaunchKernelGGL(kc_wgrad_first, dim3(nch), dim3(256), 0, h->stream, h->nx, h->ny, h->nz, total, WCHUNK,
+                       (const float *)h->xin, dout, h->wpart, h->bpart);
+    hipLaunchKernelGGL((kc_grad_reduce<true>), dim3(C * C / 256 + 1), dim3(256), 0, h->stream, nch,
+                       (const float *)h->wpart, (const float *)h->bpart, gw, gb);
+    CN_LAUNCH(h);
+    return PLSQR_OK;
+}
+
+// loss of zout against tgt/tn (batch samples), dz1 = its gradient; *loss on the host
 int loss_and_grad(plsqr_cnn *h, int batch, double *loss) {
     hipLaunchKernelGGL(kc_loss, dim3(LOSS_BLK, batch), dim3(256), 0, h->stream, h->V, batch, LOSS_BLK,
-                       (const float *)h->zout, (const float *)h->tgt, (const float *)h->tn, h->dz[0], h->lpart);
+                       (const float *)h->zout, (const float *)h->tgt, (const float *)h->tn, h->dz1, h->lpart);
     CN_LAUNCH(h);
     std::vector<float> part((size_t)batch * LOSS_BLK), tn((size_t)batch);
     CN_TRY(h, hipMemcpyAsync(part.data(), h->lpart, sizeof(float) * part.size(), hipMemcpyDeviceToHost, h->stream));
@@ -258,15 +246,26 @@ int backward(plsqr_cnn *h, int batch) {
     int cur = 0, rc;
     for (int l = LAYERS - 1; l >= 0; --l) {
         float *gw = h->grads + (size_t)l * LSZ;
-        if ((rc = wgrad(h, h->nx, h->ny, h->nz, total, h->act[l], h->dz[cur], gw, gw + WSZ, h->wpart, h->bpart,
-                        h->stream)))
-            return rc;
-        if (l > 0) {  // gradient of the layer's input, through the ReLU of layer l-1
+        const bool last = l == LAYERS - 1;
+        if (last)
+            rc = wgrad<true>(h, h->nx, h->ny, h->nz, total, h->act[l], h->dz1, gw, gw + WSZ, h->wpart, h->bpart, h->stream);
+        else if (l > 0)
+            rc = wgrad<false>(h, h->nx, h->ny, h->nz, total, h->act[l], h->dz[cur], gw, gw + WSZ, h->wpart, h->bpart,
+                              h->stream);
+        else
+            rc = wgrad_first(h, total, h->dz[cur], gw, gw + WSZ);
+        if (rc) return rc;
+        if (l == 0) break;
+        // gradient of the layer's input, through the ReLU of layer l-1
+        if (last) {
+            conv<CONV_ONE, false, CONV_BF16>(h->nx, h->ny, h->nz, batch, h->dz1, h->wb[l], nullptr, h->act[l], 0, h->dz[cur],
+                                             h->stream);
+        } else {
             conv<CONV_BF16, false, CONV_BF16>(h->nx, h->ny, h->nz, batch, h->dz[cur], h->wb[l], nullptr, h->act[l], 0,
                                               h->dz[1 - cur], h->stream);
-            CN_LAUNCH(h);
             cur = 1 - cur;
         }
+        CN_LAUNCH(h);
     }
     return PLSQR_OK;
 }
@@ -401,20 +400,21 @@ int plsqr_cnn_create(int nx, int ny, int nz, int max_batch, unsigned long long s
     hipError_t e = hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking);
     if (e != hipSuccess) return fail(set_err(h, PLSQR_ERR_HIP, std::string("hipStreamCreate: ") + hipGetErrorString(e)));
     const long long total = (long long)max_batch * h->V;
-    const int nch = (int)((total + WCHUNK - 1) / WCHUNK), nb = (int)((total + BCHUNK - 1) / BCHUNK);
+    const int nch = (int)((total + WCHUNK - 1) / WCHUNK);
     int rc;
     if ((rc = calloc_dev(h, &h->params, NPARAM)) || (rc = calloc_dev(h, &h->grads, NPARAM)) ||
         (rc = calloc_dev(h, &h->adam_m, NPARAM)) || (rc = calloc_dev(h, &h->adam_v, NPARAM)) ||
-        (rc = calloc_dev(h, &h->mask, NPARAM)) || (rc = calloc_dev(h, &h->zout, (size_t)total * C)) ||
+        (rc = calloc_dev(h, &h->mask, NPARAM)) || (rc = calloc_dev(h, &h->zout, (size_t)total)) ||
+        (rc = calloc_dev(h, &h->dz1, (size_t)total)) ||
         (rc = calloc_dev(h, &h->dz[0], (size_t)total * C)) || (rc = calloc_dev(h, &h->dz[1], (size_t)total * C)) ||
-        (rc = calloc_dev(h, &h->wpart, (size_t)nch * TAPS * C * C)) || (rc = calloc_dev(h, &h->bpart, (size_t)nb * C)) ||
+        (rc = calloc_dev(h, &h->wpart, (size_t)nch * TAPS * C * C)) || (rc = calloc_dev(h, &h->bpart, (size_t)nch * C)) ||
         (rc = calloc_dev(h, &h->lpart, (size_t)max_batch * LOSS_BLK)) || (rc = calloc_dev(h, &h->xin, (size_t)total)) ||
         (rc = calloc_dev(h, &h->tgt, (size_t)total)) || (rc = calloc_dev(h, &h->tn, (size_t)max_batch)) ||
         (rc = calloc_dev(h, &h->x0, (size_t)total)))
         return fail(rc);
     for (int l = 0; l < LAYERS; ++l)
         if ((rc = calloc_dev(h, &h->wf[l], WSZ)) || (rc = calloc_dev(h, &h->wb[l], WSZ)) ||
-            (rc = calloc_dev(h, &h->act[l], (size_t)total * C)))
+            (l > 0 && (rc = calloc_dev(h, &h->act[l], (size_t)total * C))))
             return fail(rc);
     // He initialisation (fan-in = 27 x real input channels), zero biases
     std::vector<float> p((size_t)NPARAM, 0.f);
@@ -573,18 +573,18 @@ int plsqr_cnn_predict(plsqr_cnn *h, int count, const double *atb, double *x0) {
     int rc;
     if ((rc = check(h))) return rc;
     if (count < 0 || (count > 0 && (!atb || !x0))) return set_err(h, PLSQR_ERR_ARG, "atb and x0 are required");
-    std::vector<float> z((size_t)h->V * C);
+    std::vector<float> z((size_t)h->V);
     for (int s0 = 0; s0 < count; s0 += h->max_batch) {
         const int nb = std::min(h->max_batch, count - s0);
         std::vector<double> scales;
         if ((rc = load_samples(h, nb, atb + (size_t)s0 * h->V, nullptr, &scales)) || (rc = forward(h, nb))) return rc;
         for (int s = 0; s < nb; ++s) {
-            CN_TRY(h, hipMemcpyAsync(z.data(), h->zout + (size_t)s * h->V * C, sizeof(float) * z.size(),
+            CN_TRY(h, hipMemcpyAsync(z.data(), h->zout + (size_t)s * h->V, sizeof(float) * z.size(),
                                      hipMemcpyDeviceToHost, h->stream));
             CN_TRY(h, hipStreamSynchronize(h->stream));
             double *o = x0 + (size_t)(s0 + s) * h->V;
             const double f = scales[(size_t)s] * (double)h->gain;
-            for (int v = 0; v < h->V; ++v) o[v] = f * (double)z[(size_t)v * C];
+            for (int v = 0; v < h->V; ++v) o[v] = f * (double)z[(size_t)v];
         }
     }
     return PLSQR_OK;
@@ -664,7 +664,7 @@ int plsqr_cnn_conv_backward(int nx, int ny, int nz, int batch, const float *in, 
     const long long total = (long long)batch * nx * ny * nz;
     plsqr_cnn tmp;
     plsqr_cnn *h = &tmp;
-    const int nch = (int)((total + WCHUNK - 1) / WCHUNK), nb = (int)((total + BCHUNK - 1) / BCHUNK);
+    const int nch = (int)((total + WCHUNK - 1) / WCHUNK);
     float *fin = nullptr, *fw = nullptr, *fdo = nullptr, *fdi = nullptr, *gw = nullptr, *wpart = nullptr, *bpart = nullptr;
     uint16_t *bin = nullptr, *bdo = nullptr, *wf = nullptr, *wb = nullptr;
     int rc;
@@ -675,7 +675,7 @@ int plsqr_cnn_conv_backward(int nx, int ny, int nz, int batch, const float *in, 
     if ((rc = calloc_dev(h, &fin, (size_t)total * C)) || (rc = calloc_dev(h, &fw, WSZ)) ||
         (rc = calloc_dev(h, &fdo, (size_t)total * C)) || (rc = calloc_dev(h, &fdi, (size_t)total * C)) ||
         (rc = calloc_dev(h, &gw, LSZ)) || (rc = calloc_dev(h, &wpart, (size_t)nch * TAPS * C * C)) ||
-        (rc = calloc_dev(h, &bpart, (size_t)nb * C)) || (rc = calloc_dev(h, &bin, (size_t)total * C)) ||
+        (rc = calloc_dev(h, &bpart, (size_t)nch * C)) || (rc = calloc_dev(h, &bin, (size_t)total * C)) ||
         (rc = calloc_dev(h, &bdo, (size_t)total * C)) || (rc = calloc_dev(h, &wf, WSZ)) || (rc = calloc_dev(h, &wb, WSZ))) {
         g_cnn_err = tmp.err;
         cleanup();
@@ -690,7 +690,7 @@ int plsqr_cnn_conv_backward(int nx, int ny, int nz, int batch, const float *in, 
         hipLaunchKernelGGL(kc_to_bf16, dim3(g), dim3(256), 0, 0, total * C, (const float *)fdo, bdo);
         hipLaunchKernelGGL(kc_prep_weights, dim3((WSZ + 255) / 256), dim3(256), 0, 0, (const float *)fw, wf, wb);
         conv<CONV_BF16, false, CONV_F32>(nx, ny, nz, batch, bdo, wb, nullptr, nullptr, 0, fdi, 0);
-        rc = wgrad(h, nx, ny, nz, total, bin, bdo, gw, gw + WSZ, wpart, bpart, 0);
+        rc = wgrad<false>(h, nx, ny, nz, total, bin, bdo, gw, gw + WSZ, wpart, bpart, 0);
         e = hipGetLastError();
         if (e == hipSuccess) e = hipDeviceSynchronize();
         if (e == hipSuccess) e = hipMemcpy(din, fdi, sizeof(float) * total * C, hipMemcpyDeviceToHost);

@@ -66,12 +66,12 @@ def test_conv_noalloc_takes_any_float_pointers(P, gpu_available, how):
     assert np.array_equal(out[off:].cpu().numpy().reshape(x.shape), want)
 
 
-# lines that leave few rows per sub-block (260), one line group per workgroup
-# only (410), none (600), and enough chunks of 4096 rows for nine taps each;
-# ragged last chunks.  Each weight is a sum of up to 720k products in chains of
-# 128 steps and 176 chunks: 2^-24 sqrt(300) of the result, well below 1e-5.
+# three taps per workgroup on short, long and single-voxel lines, and enough
+# chunks of 4096 rows for nine, up to the longest line that takes them (191);
+# ragged last chunks.  Each weight is a sum of up to 724k products in chains of
+# 128 steps and 177 chunks: 2^-24 sqrt(300) of the result, well below 1e-5.
 @pytest.mark.parametrize("grid,batch", [((260, 3, 3), 1), ((410, 3, 2), 2), ((600, 2, 2), 1), ((1, 70, 1), 2),
-                                        ((20, 200, 181), 1)])
+                                        ((20, 200, 181), 1), ((191, 61, 62), 1)])
 def test_weight_gradient_layouts(P, gpu_available, grid, batch):
     print(f"weight gradient: grid {grid}, batch {batch}", flush=True)
     x, w, _, d = operands(grid, batch, 8)
