@@ -165,6 +165,16 @@ int build_batch_plan(const plsqr_system *const *systems, const plsqr_grid *grids
     plan->P = P;
     plan->TW = TW;
     plan->prob.assign((size_t)P, ProblemLayout());
+    // Nonzeros per item: 4096 keep the chip's workgroups even without making
+    // the slices' partial sums a large share of mode 2 (FP64, four right-hand
+    // sides, us per iteration: 8 grids of 20^3..40^3, 113M nonzeros, 8300 per
+    // item 1717, 4700 1481, 2400 1535; 24 grids of 20^3..48^3, 675M, 8400 7851,
+    // 4200 7737).  Small batches take smaller items, down to 1024, so that
+    // there are 4096 of them (6 grids of 12^3..24^3, 11.6M nonzeros: 864 items
+    // 559, 3800 items 297, 7300 items 281).
+    long long total_nnz = 0;
+    for (int p = 0; p < P; ++p) total_nnz += systems[p] ? std::max(0LL, (long long)systems[p]->nnz_k) : 0;
+    const long long item_nnz = std::min(4096LL, std::max(1024LL, total_nnz / 4096));
     int rc;
     for (int p = 0; p < P; ++p) {
         const plsqr_system *s = systems[p];
@@ -192,8 +202,12 @@ int build_batch_plan(const plsqr_system *const *systems, const plsqr_grid *grids
             tiles.push_back(s->n);
         }
         order_tile_columns(s, tiles, perm);
-        // row slices balanced by nonzeros, about slice_rows rows each
-        const int S = std::max(1, std::min(64, (s->m_k + std::max(slice_rows, 1) - 1) / std::max(slice_rows, 1)));
+        // row slices balanced by nonzeros: at most about slice_rows rows each,
+        // and about item_nnz nonzeros per (tile, slice) item
+        const int T = (int)tiles.size() - 1;
+        const long long by_rows = (s->m_k + std::max(slice_rows, 1) - 1) / std::max(slice_rows, 1);
+        const long long by_nnz = s->nnz_k / (T * item_nnz);
+        const int S = (int)std::max(1LL, std::min({64LL, std::max(by_rows, by_nnz), (long long)s->m_k}));
         auto cut_slices = [S](const plsqr_system *q_s) {
             std::vector<int> sl((size_t)S + 1, 0);
             std::vector<long long> cnt((size_t)q_s->m_k + 1, 0);

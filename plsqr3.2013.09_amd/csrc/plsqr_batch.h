@@ -260,7 +260,7 @@ __global__ __launch_bounds__(BS) void kb_seg(const int *__restrict__ blk_item, c
     constexpr int G = 64;
     constexpr int NWV = BS / G;
     static_assert(G == kWave, "one segment group per wavefront");
-    __shared__ T xl[128 * K];
+    __shared__ __align__(16) T xl[128 * K];
     __shared__ __align__(16) T lv[NWV][CH + 8];
     __shared__ __align__(16) uint8_t lx[NWV][CH + 8];
     const int it = blk_item[blockIdx.x];
@@ -302,11 +302,23 @@ __global__ __launch_bounds__(BS) void kb_seg(const int *__restrict__ blk_item, c
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
             const int e0 = beg > q0 ? beg : q0;
             const int e1 = end < q0 + cnt ? end : q0 + cnt;
-            for (int e = e0; e < e1; ++e) {
-                const T a = bv[sh + e];
-                const T *xv = xl + (int)bx[sh + e] * K;
+            // two entries per step, their LDS reads in flight together, added
+            // in entry order
+            int e = e0;
+            for (; e + 1 < e1; e += 2) {
+                const T a0 = bv[sh + e], a1 = bv[sh + e + 1];
+                const VK<T, K> x0 = ldk<T, K>(xl, (size_t)bx[sh + e]), x1 = ldk<T, K>(xl, (size_t)bx[sh + e + 1]);
 #pragma unroll
-                for (int k = 0; k < K; ++k) acc[k].add(a, xv[k]);
+                for (int k = 0; k < K; ++k) {
+                    acc[k].add(a0, x0.a[k]);
+                    acc[k].add(a1, x1.a[k]);
+                }
+            }
+            if (e < e1) {
+                const T a = bv[sh + e];
+                const VK<T, K> xv = ldk<T, K>(xl, (size_t)bx[sh + e]);
+#pragma unroll
+                for (int k = 0; k < K; ++k) acc[k].add(a, xv.a[k]);
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
@@ -575,20 +587,40 @@ __global__ __launch_bounds__(BS) void kb_combine(int ncc, const int *__restrict_
         for (int k = 0; k < K; ++k) ssq[k] = 0.0;
         for (int c = cc_col[ch] + threadIdx.x; c < cc_col[ch + 1]; c += BS) {
             const long long cl = c - cb;
+            // the slices, then the damping entries, four loads in flight at a
+            // time (past the end: the last one again, dropped)
             VK<double, K> tk = ldk<double, K>(P, (size_t)(pb + cl));
-            for (int q = 1; q < S; ++q) {
-                const VK<double, K> t2 = ldk<double, K>(P, (size_t)(pb + (long long)q * n + cl));
+            for (int q = 1; q < S; q += 4) {
+                VK<double, K> t2[4];
 #pragma unroll
-                for (int k = 0; k < K; ++k) tk.a[k] += t2.a[k];
+                for (int i = 0; i < 4; ++i)
+                    t2[i] = ldk<double, K>(P, (size_t)(pb + (long long)min(q + i, S - 1) * n + cl));
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+                        if (q + i < S) tk.a[k] += t2[i].a[k];
             }
             double td[K];
 #pragma unroll
             for (int k = 0; k < K; ++k) td[k] = 0.0;
-            for (int e = dcp[c]; e < dcp[c + 1]; ++e) {
-                const VK<T, K> q = ldk<T, K>(u, (size_t)dri[e]);
-                const double d = dcv[e];
+            const int de = dcp[c + 1];
+            for (int e = dcp[c]; e < de; e += 4) {
+                int r[4];
+                double d[4];
+                VK<T, K> q[4];
 #pragma unroll
-                for (int k = 0; k < K; ++k) td[k] += d * ((double)q.a[k] * ib[k]);
+                for (int i = 0; i < 4; ++i) {
+                    r[i] = dri[min(e + i, de - 1)];
+                    d[i] = dcv[min(e + i, de - 1)];
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) q[i] = ldk<T, K>(u, (size_t)r[i]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int k = 0; k < K; ++k)
+                        if (e + i < de) td[k] += d[i] * ((double)q[i].a[k] * ib[k]);
             }
             VK<T, K> vv = ldk<T, K>(v, (size_t)c);
             if (cs) {
