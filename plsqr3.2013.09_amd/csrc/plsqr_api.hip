@@ -871,8 +871,12 @@ int build(plsqr_op *op, const plsqr_system *s, const std::vector<int> &hb, const
             }
             // chunks of at most rt_chunk groups (PLSQR_M1_CHUNK, 0: whole
             // items), dealt so that chunk 8k + s belongs to row slice s and
-            // runs on the XCD of the slice's other work
-            op->rt_chunk = std::max(0, env_int("PLSQR_M1_CHUNK", 16));
+            // runs on the XCD of the slice's other work: 16 groups where that
+            // makes four workgroups per CU, else fewer, down to one group per
+            // wavefront (16^3 / 20k rays, 1.1k groups: pass 1 13.3 us in chunks
+            // of 16, four rounds of loads one after another; CHUNK_US in 4s)
+            const int per_cu = (int)(R->n_grp / (4LL * op->cu));
+            op->rt_chunk = std::max(0, env_int("PLSQR_M1_CHUNK", std::min(16, std::max(4, per_cu / 4 * 4))));
             if (op->rt_chunk > 0) {
                 const int S = L1->S;
                 std::vector<std::vector<int>> ci((size_t)S), cg((size_t)S);

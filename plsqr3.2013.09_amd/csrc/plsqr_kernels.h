@@ -111,7 +111,9 @@ __device__ __forceinline__ void dot32_add(double &acc, float a, double x) { acc 
 // A damping row's entries b .. e-1 (1 to 3 for the grid stencils), four at a
 // time: the column indices and values, then the x gathers in flight
 // together, added in entry order as acc += a * x (FP64 values) or as
-// dot32_add (FP32 values, the exact product).
+// dot32_add (FP32 values, the exact product).  Past the end the first entry is
+// loaded again and dropped: a load that is not issued for some lanes waits for
+// itself.
 template <class A, class X>
 __device__ __forceinline__ double damp_row_sum(int b, int e, const int *__restrict__ ci, const A *__restrict__ av,
                                                const X *__restrict__ x) {
@@ -122,12 +124,12 @@ __device__ __forceinline__ double damp_row_sum(int b, int e, const int *__restri
         X g[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const bool on = k0 + j < e;
-            i[j] = on ? ci[k0 + j] : 0;
-            a[j] = on ? av[k0 + j] : A(0);
+            const int k = k0 + j < e ? k0 + j : b;
+            i[j] = ci[k];
+            a[j] = av[k];
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) g[j] = k0 + j < e ? x[i[j]] : X(0);
+        for (int j = 0; j < 4; ++j) g[j] = x[i[j]];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             if (k0 + j < e) {

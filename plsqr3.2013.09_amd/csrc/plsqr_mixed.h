@@ -211,18 +211,20 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_combine32(int m_k, int m, int
     for (int g = blockIdx.x / S; g < groups; g += gridDim.x / S) {
         const int r = r0 + g * R + slot;
         double acc = 0.0;
+        const float yo = y[min(r, r1 - 1)];  // in flight with the partials
         if (r < r1) acc = ray_partials<LC>(ray_seg, segv, ray_ptr[r], ray_ptr[r + 1], lane);
         acc = group_sum<LC>(acc);
         if (lane == 0 && r < r1) {
-            const float yn = (y[r] * s1) * s2 + (float)acc;
+            const float yn = (yo * s1) * s2 + (float)acc;
             y[r] = yn;
             ssq_k += (double)yn * (double)yn;
         }
     }
     for (long long r = (long long)m_k + (long long)blockIdx.x * BS + threadIdx.x; r < m;
          r += (long long)gridDim.x * BS) {
+        const float yo = y[r];
         const double acc = damp_row_sum(rp[r], rp[r + 1], ci, av, x);
-        const float yn = (y[r] * s1) * s2 + (float)acc;
+        const float yn = (yo * s1) * s2 + (float)acc;
         y[r] = yn;
         ssq_d += (double)yn * (double)yn;
     }
@@ -414,8 +416,8 @@ __global__ __launch_bounds__(BS) void k_cols_combine32(int n, int m_k, int nsl, 
     const float *ud = u + m_k;
     double ssq = 0.0;
     for (int c = blockIdx.x * BS + threadIdx.x; c < n; c += gridDim.x * BS) {
-        double tk = P[c];
-        for (int s = 1; s < nsl; ++s) tk += P[(size_t)s * n + c];
+        const float vc = v[c];
+        const double tk = slice_sum(P, n, c, nsl);
         double td = 0.0;
         if (dlen) {  // damping columns interleaved by groups of 64 (k_cols_combine)
             td = damp_col_sum_il(dlen[c], dcp[c], dri, dav, ud, ib);
@@ -424,12 +426,12 @@ __global__ __launch_bounds__(BS) void k_cols_combine32(int n, int m_k, int nsl, 
         }
         if (cs) {
             const double d = cs[c];
-            const float vn = v[c] * vs + (float)(d * d * (tk + td));
+            const float vn = vc * vs + (float)(d * d * (tk + td));
             v[c] = vn;
             const double q = (double)vn / d;
             ssq += q * q;
         } else {
-            const float vn = v[c] * vs + (float)(tk + td);
+            const float vn = vc * vs + (float)(tk + td);
             v[c] = vn;
             ssq += (double)vn * (double)vn;
         }

@@ -272,10 +272,10 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_combine(int m_k, int m, int S
     for (int g = blockIdx.x / S; g < groups; g += gridDim.x / S) {
         const int r = r0 + g * R + slot;
         double acc = 0.0;
+        double yn = y[min(r, r1 - 1)];  // in flight with the partials
         if (r < r1) acc = ray_partials<LC>(ray_seg, segv, ray_ptr[r], ray_ptr[r + 1], lane);
         acc = group_sum<LC>(acc);
         if (lane == 0 && r < r1) {
-            double yn = y[r];
             if (scaled) yn = (yn * s1) * s2;
             yn = yn + acc;
             y[r] = yn;
@@ -284,8 +284,8 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_combine(int m_k, int m, int S
     }
     for (long long r = (long long)m_k + (long long)blockIdx.x * BS + threadIdx.x; r < m;
          r += (long long)gridDim.x * BS) {
-        const double acc = damp_row_sum(rp[r], rp[r + 1], ci, av, x);
         double yn = y[r];
+        const double acc = damp_row_sum(rp[r], rp[r + 1], ci, av, x);
         if (scaled) yn = (yn * s1) * s2;
         yn = yn + acc;
         y[r] = yn;
@@ -678,7 +678,7 @@ __global__ void k_remap(long long len, const int *__restrict__ map, int *__restr
 
 // Interleaved damping column: its len entries at q, q + 64, ..., four at a
 // time (their indices and values, then the four u gathers in flight
-// together), added in entry order.
+// together), added in entry order.  Past the end slot 0 is loaded and dropped.
 template <class U>
 __device__ __forceinline__ double damp_col_sum_il(int len, int q, const int *__restrict__ dri,
                                                   const double *__restrict__ dav, const U *__restrict__ ud, double ib) {
@@ -688,17 +688,32 @@ __device__ __forceinline__ double damp_col_sum_il(int len, int q, const int *__r
         double a[4], g[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const bool on = k0 + j < len;
-            i[j] = on ? dri[q + j * kWave] : 0;
-            a[j] = on ? dav[q + j * kWave] : 0.0;
+            const int k = k0 + j < len ? q + j * kWave : 0;
+            i[j] = dri[k];
+            a[j] = dav[k];
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) g[j] = k0 + j < len ? (double)ud[i[j]] : 0.0;
+        for (int j = 0; j < 4; ++j) g[j] = (double)ud[i[j]];
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (k0 + j < len) td += a[j] * (g[j] * ib);
     }
     return td;
+}
+
+// Column c's slice partials added in slice order, eight loads in flight (past
+// the last slice: that one again, dropped).
+__device__ __forceinline__ double slice_sum(const double *__restrict__ P, int n, int c, int nsl) {
+    double tk = P[c];
+    for (int s = 1; s < nsl; s += 8) {
+        double p[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p[j] = P[(size_t)min(s + j, nsl - 1) * n + c];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (s + j < nsl) tk += p[j];
+    }
+    return tk;
 }
 
 // v[c] <- fl(v[c]*vscale) + (tk + td) with tk the slice partials summed in
@@ -747,10 +762,9 @@ __global__ __launch_bounds__(BS) void k_cols_combine(int n, int m_k, int nsl,
     const double *ud = u + m_k;
     double ssq = 0.0;
     for (int c = blockIdx.x * BS + threadIdx.x; c < n; c += gridDim.x * BS) {
-        double tk = P[c];
-        for (int s = 1; s < nsl; ++s) tk += P[(size_t)s * n + c];
-        const double td = damp_col_sum(c, dcp, dlen, dri, dav, ud, ib);
         double vn = v[c];
+        const double tk = slice_sum(P, n, c, nsl);
+        const double td = damp_col_sum(c, dcp, dlen, dri, dav, ud, ib);
         if (scaled) vn = vn * vs;
         if (cs) {
             const double d = cs[c];
