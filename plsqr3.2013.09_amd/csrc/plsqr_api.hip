@@ -306,18 +306,29 @@ void launch_pass1(plsqr_op *op, const T *val, const T *x, const Scal *sc, T *seg
 #undef PASS1
 }
 
-int launch_rows(plsqr_op *op, const double *x, double *y, const Scal *sc, double *part) {
+// yp: NULL, or y is in the caller's order, row r at y[yp[r]] (tiled rows only)
+int launch_rows(plsqr_op *op, const double *x, double *y, const Scal *sc, double *part, const int *yp = nullptr) {
     using namespace plsqr;
     dim3 g(op->G1), b(BS);
     if (op->rtiled) {
         launch_pass1<double>(op, op->rt_val, x, sc, op->rt_segv);
         LAUNCH_CHECK(op);
+#define COMB(LC, EXT)                                                                                                 \
+    hipLaunchKernelGGL((k_rows_tiled_combine<LC, BS, EXT>), g, b, 0, op->stream, op->m_k, op->m, op->tS, op->bounds,  \
+                       op->rt_rptr, op->rt_rseg, op->rt_segv, op->rp, op->ci, op->rv, x, y, sc, part, yp)
+#define COMB_LC(LC)       \
+    if (yp)               \
+        COMB(LC, true);   \
+    else                  \
+        COMB(LC, false);
         switch (op->rt_lc) {
-            case 1: hipLaunchKernelGGL((k_rows_tiled_combine<1, BS>), g, b, 0, op->stream, op->m_k, op->m, op->tS, op->bounds, op->rt_rptr, op->rt_rseg, op->rt_segv, op->rp, op->ci, op->rv, x, y, sc, part); break;
-            case 2: hipLaunchKernelGGL((k_rows_tiled_combine<2, BS>), g, b, 0, op->stream, op->m_k, op->m, op->tS, op->bounds, op->rt_rptr, op->rt_rseg, op->rt_segv, op->rp, op->ci, op->rv, x, y, sc, part); break;
-            case 8: hipLaunchKernelGGL((k_rows_tiled_combine<8, BS>), g, b, 0, op->stream, op->m_k, op->m, op->tS, op->bounds, op->rt_rptr, op->rt_rseg, op->rt_segv, op->rp, op->ci, op->rv, x, y, sc, part); break;
-            default: hipLaunchKernelGGL((k_rows_tiled_combine<4, BS>), g, b, 0, op->stream, op->m_k, op->m, op->tS, op->bounds, op->rt_rptr, op->rt_rseg, op->rt_segv, op->rp, op->ci, op->rv, x, y, sc, part); break;
+            case 1: COMB_LC(1) break;
+            case 2: COMB_LC(2) break;
+            case 8: COMB_LC(8) break;
+            default: COMB_LC(4) break;
         }
+#undef COMB_LC
+#undef COMB
         LAUNCH_CHECK(op);
         return PLSQR_OK;
     }
@@ -364,9 +375,10 @@ int launch_residual(plsqr_op *op, const double *x, const double *b, double *r) {
 
 
 // cs: column scales of an LSQR on A D (the FP64 inner iteration of a scaled
-// solve), NULL for A itself
+// solve), NULL for A itself; vp: NULL, or v is in the caller's order, column c
+// at v[vp[c]] (tiled columns only)
 int launch_cols(plsqr_op *op, const double *u, double *v, const Scal *sc, double *part,
-                const double *cs = nullptr) {
+                const double *cs = nullptr, const int *vp = nullptr) {
     using namespace plsqr;
     if (op->tiled) {
         const SlotRows sr{op->t_pvox, op->t_rbase, op->t_roff};
@@ -395,9 +407,14 @@ int launch_cols(plsqr_op *op, const double *u, double *v, const Scal *sc, double
         }
 #undef COLS
         LAUNCH_CHECK(op);
-        hipLaunchKernelGGL((k_cols_combine<BS>), dim3(op->G4), dim3(BS), 0, op->stream, op->n, op->m_k, op->tS,
-                           op->P, dcol_start(op), dcol_row(op), dcol_val(op), u, sc, v, part, cs,
-                           (const uint8_t *)op->dlen);
+        if (vp)
+            hipLaunchKernelGGL((k_cols_combine<BS, true>), dim3(op->G4), dim3(BS), 0, op->stream, op->n, op->m_k,
+                               op->tS, op->P, dcol_start(op), dcol_row(op), dcol_val(op), u, sc, v, part, cs,
+                               (const uint8_t *)op->dlen, vp);
+        else
+            hipLaunchKernelGGL((k_cols_combine<BS>), dim3(op->G4), dim3(BS), 0, op->stream, op->n, op->m_k, op->tS,
+                               op->P, dcol_start(op), dcol_row(op), dcol_val(op), u, sc, v, part, cs,
+                               (const uint8_t *)op->dlen);
         LAUNCH_CHECK(op);
         return PLSQR_OK;
     }
@@ -548,18 +565,24 @@ int b_internal(plsqr_op *op, const double *b, const double **out) {
 }
 
 // aprod on operands each either in the caller's order (renumbered in and,
-// for the output, back) or already in the device order
+// for the output, back) or already in the device order.  The tiled operator's
+// combines update a caller-order output in place.
 int aprod_any(plsqr_op *op, int mode, double *x, bool x_ext, double *y, bool y_ext) {
     int rc;
+    const bool tiled = mode == 1 ? op->rtiled : op->tiled;
+    const bool move_x = x_ext && op->permuted, move_y = y_ext && op->rowperm;
+    const bool place_x = mode == 2 && tiled && move_x, place_y = mode == 1 && tiled && move_y;
     double *xi = x, *yi = y;
-    if (x_ext && op->permuted) {
+    if (move_x && !place_x) {
         if ((rc = to_internal(op, x, op->hx2))) return rc;
         xi = op->hx2;
     }
-    if (y_ext && op->rowperm) {
+    if (move_y && !place_y) {
         if ((rc = rows_to_internal(op, y, op->hy2))) return rc;
         yi = op->hy2;
     }
+    if (place_x) return launch_cols(op, yi, x, nullptr, nullptr, nullptr, op->inv);
+    if (place_y) return launch_rows(op, xi, y, nullptr, nullptr, op->rperm);
     if ((rc = mode == 1 ? aprod1_dev(op, xi, yi) : aprod2_dev(op, xi, yi))) return rc;
     if (mode == 2 && xi != x) return to_external(op, xi, x);
     if (mode == 1 && yi != y) return rows_to_external(op, yi, y);
@@ -874,7 +897,7 @@ int build(plsqr_op *op, const plsqr_system *s, const std::vector<int> &hb, const
             // runs on the XCD of the slice's other work: 16 groups where that
             // makes four workgroups per CU, else fewer, down to one group per
             // wavefront (16^3 / 20k rays, 1.1k groups: pass 1 13.3 us in chunks
-            // of 16, four rounds of loads one after another; CHUNK_US in 4s)
+            // of 16, four rounds of loads one after another; 6.6 in 4s)
             const int per_cu = (int)(R->n_grp / (4LL * op->cu));
             op->rt_chunk = std::max(0, env_int("PLSQR_M1_CHUNK", std::min(16, std::max(4, per_cu / 4 * 4))));
             if (op->rt_chunk > 0) {
@@ -1321,38 +1344,50 @@ static void launch_cols_tiled32(plsqr_op *op, const float *u, const Scal *sc) {
 #undef COLS32
 }
 
-// FP32 aprod on internal-order vectors (x: n, y: m floats) with the plain Scal
-// FP32 per-ray combine with rt_lc lanes per ray
-static void launch_combine32(plsqr_op *op, const float *x, float *y, const plsqr::Scal *sc) {
+// FP32 per-ray combine with rt_lc lanes per ray; yp as in launch_rows
+static void launch_combine32(plsqr_op *op, const float *x, float *y, const plsqr::Scal *sc, const int *yp = nullptr) {
     using namespace plsqr;
-#define COMB32(LC)                                                                                                 \
-    hipLaunchKernelGGL((k_rows_tiled_combine32<LC, BS>), dim3(op->G1), dim3(BS), 0, op->stream, op->m_k, op->m,  \
-                       op->tS, op->bounds, op->rt_rptr, op->rt_rseg, (const float *)op->rt_segv, op->rp, op->ci,  \
-                       op->rv32, x, y, sc, op->part)
+#define COMB32(LC, EXT)                                                                                              \
+    hipLaunchKernelGGL((k_rows_tiled_combine32<LC, BS, EXT>), dim3(op->G1), dim3(BS), 0, op->stream, op->m_k, op->m, \
+                       op->tS, op->bounds, op->rt_rptr, op->rt_rseg, (const float *)op->rt_segv, op->rp, op->ci,    \
+                       op->rv32, x, y, sc, op->part, yp)
+#define COMB32_LC(LC)     \
+    if (yp)               \
+        COMB32(LC, true); \
+    else                  \
+        COMB32(LC, false);
     switch (op->rt_lc) {
-        case 2: COMB32(2); break;
-        case 8: COMB32(8); break;
-        default: COMB32(4); break;
+        case 2: COMB32_LC(2) break;
+        case 8: COMB32_LC(8) break;
+        default: COMB32_LC(4) break;
     }
+#undef COMB32_LC
 #undef COMB32
 }
 
-static int aprod32_internal(plsqr_op *op, int mode, float *x, float *y) {
+// FP32 aprod on internal-order vectors (x: n, y: m floats) with the plain
+// Scal; yp, vp: the output is in the caller's order (launch_rows, launch_cols)
+static int aprod32_internal(plsqr_op *op, int mode, float *x, float *y, const int *yp = nullptr, const int *vp = nullptr) {
     using namespace plsqr;
     const Scal *sp = op->sc_plain;
     if (mode == 1) {
         if (op->rtiled) {
             launch_pass1<float>(op, op->rt_val32, x, sp, (float *)op->rt_segv);
-            launch_combine32(op, x, y, sp);
+            launch_combine32(op, x, y, sp, yp);
         } else {
             hipLaunchKernelGGL((k_rows32<16, BS>), dim3(op->G1), dim3(BS), 0, op->stream, op->m_k, op->m, op->rp,
                                op->ci, op->rv32, x, y, sp, op->part);
         }
     } else {
         launch_cols_tiled32(op, y, sp);
-        hipLaunchKernelGGL((k_cols_combine32<BS>), dim3(op->G4), dim3(BS), 0, op->stream, op->n, op->m_k, op->tS,
-                           op->P, dcol_start(op), dcol_row(op), dcol_val(op), y, sp, x, op->part,
-                           (const double *)nullptr, (const uint8_t *)op->dlen);
+        if (vp)
+            hipLaunchKernelGGL((k_cols_combine32<BS, true>), dim3(op->G4), dim3(BS), 0, op->stream, op->n, op->m_k,
+                               op->tS, op->P, dcol_start(op), dcol_row(op), dcol_val(op), y, sp, x, op->part,
+                               (const double *)nullptr, (const uint8_t *)op->dlen, vp);
+        else
+            hipLaunchKernelGGL((k_cols_combine32<BS>), dim3(op->G4), dim3(BS), 0, op->stream, op->n, op->m_k, op->tS,
+                               op->P, dcol_start(op), dcol_row(op), dcol_val(op), y, sp, x, op->part,
+                               (const double *)nullptr, (const uint8_t *)op->dlen);
     }
     LAUNCH_CHECK(op);
     return PLSQR_OK;
@@ -1383,24 +1418,27 @@ int plsqr_aprod_device_f32(plsqr_op *op, int mode, float *x_dev, float *y_dev) {
     int rc;
     if ((rc = ensure_aprod32(op))) return rc;
     const int gn = grid_for(op->n, 256, op->cu * 4), gm = grid_for(op->m, 256, op->cu * 4);
-    // caller order -> device order
-    if (op->permuted)
-        hipLaunchKernelGGL(k_gather32, dim3(gn), dim3(256), 0, op->stream, op->n, op->inv, x_dev, op->v32);
-    else
-        HIP_TRY(op, hipMemcpyAsync(op->v32, x_dev, sizeof(float) * op->n, hipMemcpyDeviceToDevice, op->stream));
-    if (op->rowperm) {
-        hipLaunchKernelGGL(k_gather32, dim3(gm), dim3(256), 0, op->stream, op->m, op->rperm, y_dev, op->u32);
-    } else {
-        HIP_TRY(op, hipMemcpyAsync(op->u32, y_dev, sizeof(float) * op->m, hipMemcpyDeviceToDevice, op->stream));
+    // caller order -> device order, except an output that a combine updates in place
+    const bool place_x = mode == 2 && op->permuted, place_y = mode == 1 && op->rowperm && op->rtiled;
+    if (!place_x) {
+        if (op->permuted)
+            hipLaunchKernelGGL(k_gather32, dim3(gn), dim3(256), 0, op->stream, op->n, op->inv, x_dev, op->v32);
+        else
+            HIP_TRY(op, hipMemcpyAsync(op->v32, x_dev, sizeof(float) * op->n, hipMemcpyDeviceToDevice, op->stream));
+    }
+    if (!place_y) {
+        if (op->rowperm)
+            hipLaunchKernelGGL(k_gather32, dim3(gm), dim3(256), 0, op->stream, op->m, op->rperm, y_dev, op->u32);
+        else
+            HIP_TRY(op, hipMemcpyAsync(op->u32, y_dev, sizeof(float) * op->m, hipMemcpyDeviceToDevice, op->stream));
     }
     LAUNCH_CHECK(op);
+    if (place_x) return aprod32_internal(op, mode, x_dev, op->u32, nullptr, op->inv);
+    if (place_y) return aprod32_internal(op, mode, op->v32, y_dev, op->rperm);
     if ((rc = aprod32_internal(op, mode, op->v32, op->u32))) return rc;
     // back to the caller's order: only the output moves
     if (mode == 2) {
-        if (op->permuted)
-            hipLaunchKernelGGL(k_gather32, dim3(gn), dim3(256), 0, op->stream, op->n, op->perm, op->v32, x_dev);
-        else
-            HIP_TRY(op, hipMemcpyAsync(x_dev, op->v32, sizeof(float) * op->n, hipMemcpyDeviceToDevice, op->stream));
+        HIP_TRY(op, hipMemcpyAsync(x_dev, op->v32, sizeof(float) * op->n, hipMemcpyDeviceToDevice, op->stream));
     } else if (op->rowperm) {
         hipLaunchKernelGGL(k_gather32, dim3(gm), dim3(256), 0, op->stream, op->m, op->rinv, op->u32, y_dev);
     } else {

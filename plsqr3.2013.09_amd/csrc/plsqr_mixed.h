@@ -189,7 +189,7 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_c32(int S, const int *__restr
 // added in tile order in FP64); damping rows and the FP64 ||y||^2 partials as in
 // k_rows32.  Workgroup b takes the rays of row slice b % S, as in
 // k_rows_tiled_combine.
-template <int LC, int BS>
+template <int LC, int BS, bool EXT = false>
 __global__ __launch_bounds__(BS) void k_rows_tiled_combine32(int m_k, int m, int S, const int *__restrict__ bounds,
                                                              const int *__restrict__ ray_ptr,
                                                              const int *__restrict__ ray_seg,
@@ -197,7 +197,8 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_combine32(int m_k, int m, int
                                                              const int *__restrict__ rp, const int *__restrict__ ci,
                                                              const float *__restrict__ av,
                                                              const float *__restrict__ x, float *__restrict__ y,
-                                                             const Scal *__restrict__ sc, double *__restrict__ part) {
+                                                             const Scal *__restrict__ sc, double *__restrict__ part,
+                                                             const int *__restrict__ yp = nullptr) {
     __shared__ double sh[BS / kWave];
     if (sc->done) return;
     const float s1 = (float)sc->ib, s2 = (float)(-sc->alpha);
@@ -211,21 +212,23 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_combine32(int m_k, int m, int
     for (int g = blockIdx.x / S; g < groups; g += gridDim.x / S) {
         const int r = r0 + g * R + slot;
         double acc = 0.0;
-        const float yo = y[min(r, r1 - 1)];  // in flight with the partials
+        const int ry = EXT ? yp[min(r, r1 - 1)] : min(r, r1 - 1);
+        const float yo = y[ry];  // in flight with the partials
         if (r < r1) acc = ray_partials<LC>(ray_seg, segv, ray_ptr[r], ray_ptr[r + 1], lane);
         acc = group_sum<LC>(acc);
         if (lane == 0 && r < r1) {
             const float yn = (yo * s1) * s2 + (float)acc;
-            y[r] = yn;
+            y[ry] = yn;
             ssq_k += (double)yn * (double)yn;
         }
     }
     for (long long r = (long long)m_k + (long long)blockIdx.x * BS + threadIdx.x; r < m;
          r += (long long)gridDim.x * BS) {
-        const float yo = y[r];
+        const long long ry = EXT ? (long long)yp[r] : r;
+        const float yo = y[ry];
         const double acc = damp_row_sum(rp[r], rp[r + 1], ci, av, x);
         const float yn = (yo * s1) * s2 + (float)acc;
-        y[r] = yn;
+        y[ry] = yn;
         ssq_d += (double)yn * (double)yn;
     }
     const double a = block_sum<BS>(ssq_k, sh);
@@ -396,7 +399,7 @@ __global__ __launch_bounds__(BS, 8) void k_cols_tiled32(
 
 // v32[c] <- fl32(v32*vscale) + (tk + td): tk the FP64 slice partials, td the
 // damping column (FP64 values, FP32 u); FP64 partial sums of squares.
-template <int BS>
+template <int BS, bool EXT = false>
 //
 // cs (may be NULL): the column scales d of LSQR on A D.  The solver then
 // keeps v^ = D v (and w^ = D w, so x += t1 w^ directly): mode 1 of A D on v
@@ -408,7 +411,8 @@ __global__ __launch_bounds__(BS) void k_cols_combine32(int n, int m_k, int nsl, 
                                                        const Scal *__restrict__ sc, float *__restrict__ v,
                                                        double *__restrict__ part,
                                                        const double *__restrict__ cs = nullptr,
-                                                       const uint8_t *__restrict__ dlen = nullptr) {
+                                                       const uint8_t *__restrict__ dlen = nullptr,
+                                                       const int *__restrict__ vp = nullptr) {
     __shared__ double sh[BS / kWave];
     if (sc->done || !sc->beta_pos) return;
     const double ib = sc->ib;
@@ -416,7 +420,8 @@ __global__ __launch_bounds__(BS) void k_cols_combine32(int n, int m_k, int nsl, 
     const float *ud = u + m_k;
     double ssq = 0.0;
     for (int c = blockIdx.x * BS + threadIdx.x; c < n; c += gridDim.x * BS) {
-        const float vc = v[c];
+        const int cv = EXT ? vp[c] : c;
+        const float vc = v[cv];
         const double tk = slice_sum(P, n, c, nsl);
         double td = 0.0;
         if (dlen) {  // damping columns interleaved by groups of 64 (k_cols_combine)
@@ -427,12 +432,12 @@ __global__ __launch_bounds__(BS) void k_cols_combine32(int n, int m_k, int nsl, 
         if (cs) {
             const double d = cs[c];
             const float vn = vc * vs + (float)(d * d * (tk + td));
-            v[c] = vn;
+            v[cv] = vn;
             const double q = (double)vn / d;
             ssq += q * q;
         } else {
             const float vn = vc * vs + (float)(tk + td);
-            v[c] = vn;
+            v[cv] = vn;
             ssq += (double)vn * (double)vn;
         }
     }

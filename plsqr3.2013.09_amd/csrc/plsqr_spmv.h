@@ -244,8 +244,11 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_c(int S, const int *__restric
 // slice b % S (bounds[s] .. bounds[s+1]), the slice whose items pass 1 ran
 // on the same XCD (item t*S + s is workgroup t*S + s there), so the partials
 // it reads were written through, and stay in, that XCD's L2.  The grid is a
-// multiple of S.
-template <int LC, int BS>
+// multiple of S.  EXT: y is in the caller's order, row r at y[yp[r]]; each
+// element is read and written by one lane, which costs the same scattered
+// accesses as one reordering pass and saves two (37 x 29 x 41 / 351k rays:
+// two launches of 8 us).
+template <int LC, int BS, bool EXT = false>
 __global__ __launch_bounds__(BS) void k_rows_tiled_combine(int m_k, int m, int S, const int *__restrict__ bounds,
                                                            const int *__restrict__ ray_ptr,
                                                            const int *__restrict__ ray_seg,
@@ -253,7 +256,8 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_combine(int m_k, int m, int S
                                                            const int *__restrict__ rp, const int *__restrict__ ci,
                                                            const double *__restrict__ av,
                                                            const double *__restrict__ x, double *__restrict__ y,
-                                                           const Scal *__restrict__ sc, double *__restrict__ part) {
+                                                           const Scal *__restrict__ sc, double *__restrict__ part,
+                                                           const int *__restrict__ yp = nullptr) {
     __shared__ double sh[BS / kWave];
     double s1 = 1.0, s2 = 1.0;
     const bool scaled = sc != nullptr;
@@ -272,23 +276,25 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_combine(int m_k, int m, int S
     for (int g = blockIdx.x / S; g < groups; g += gridDim.x / S) {
         const int r = r0 + g * R + slot;
         double acc = 0.0;
-        double yn = y[min(r, r1 - 1)];  // in flight with the partials
+        const int ry = EXT ? yp[min(r, r1 - 1)] : min(r, r1 - 1);
+        double yn = y[ry];  // in flight with the partials
         if (r < r1) acc = ray_partials<LC>(ray_seg, segv, ray_ptr[r], ray_ptr[r + 1], lane);
         acc = group_sum<LC>(acc);
         if (lane == 0 && r < r1) {
             if (scaled) yn = (yn * s1) * s2;
             yn = yn + acc;
-            y[r] = yn;
+            y[ry] = yn;
             ssq_k += yn * yn;
         }
     }
     for (long long r = (long long)m_k + (long long)blockIdx.x * BS + threadIdx.x; r < m;
          r += (long long)gridDim.x * BS) {
-        double yn = y[r];
+        const long long ry = EXT ? (long long)yp[r] : r;
+        double yn = y[ry];
         const double acc = damp_row_sum(rp[r], rp[r + 1], ci, av, x);
         if (scaled) yn = (yn * s1) * s2;
         yn = yn + acc;
-        y[r] = yn;
+        y[ry] = yn;
         ssq_d += yn * yn;
     }
     if (part) {
@@ -739,7 +745,8 @@ __device__ __forceinline__ double damp_col_sum(int c, const int *__restrict__ dc
     return td;
 }
 
-template <int BS>
+// EXT: v is in the caller's order, column c at v[vp[c]].
+template <int BS, bool EXT = false>
 __global__ __launch_bounds__(BS) void k_cols_combine(int n, int m_k, int nsl,
                                                      const double *__restrict__ P,
                                                      const int *__restrict__ dcp,
@@ -750,7 +757,8 @@ __global__ __launch_bounds__(BS) void k_cols_combine(int n, int m_k, int nsl,
                                                      double *__restrict__ v,
                                                      double *__restrict__ part,
                                                      const double *__restrict__ cs = nullptr,
-                                                     const uint8_t *__restrict__ dlen = nullptr) {
+                                                     const uint8_t *__restrict__ dlen = nullptr,
+                                                     const int *__restrict__ vp = nullptr) {
     __shared__ double sh[BS / kWave];
     double ib = 1.0, vs = 1.0;
     const bool scaled = sc != nullptr;
@@ -762,19 +770,20 @@ __global__ __launch_bounds__(BS) void k_cols_combine(int n, int m_k, int nsl,
     const double *ud = u + m_k;
     double ssq = 0.0;
     for (int c = blockIdx.x * BS + threadIdx.x; c < n; c += gridDim.x * BS) {
-        double vn = v[c];
+        const int cv = EXT ? vp[c] : c;
+        double vn = v[cv];
         const double tk = slice_sum(P, n, c, nsl);
         const double td = damp_col_sum(c, dcp, dlen, dri, dav, ud, ib);
         if (scaled) vn = vn * vs;
         if (cs) {
             const double d = cs[c];
             vn = vn + d * d * (tk + td);
-            v[c] = vn;
+            v[cv] = vn;
             const double q = vn / d;
             ssq += q * q;
         } else {
             vn = vn + (tk + td);
-            v[c] = vn;
+            v[cv] = vn;
             ssq += vn * vn;
         }
     }
