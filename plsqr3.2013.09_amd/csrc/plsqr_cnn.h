@@ -680,13 +680,31 @@ __global__ __launch_bounds__(256) void kc_wgrad_first(int nx, int ny, int nz, lo
 
 // bf16 weights of one layer: forward order wf[t][n][k] = W[t][n][k] and the
 // data-gradient order wb[t][k][n] = W[26 - t][n][k]
-__global__ void kc_prep_weights(const float *__restrict__ W, uint16_t *__restrict__ wf, uint16_t *__restrict__ wb) {
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= TAPS * C * C) return;
+__device__ __forceinline__ void put_weight(int idx, float v, uint16_t *__restrict__ wf, uint16_t *__restrict__ wb) {
     const int t = idx / (C * C), n = (idx / C) % C, k = idx % C;
-    const uint16_t h = f2bf(W[idx]);
+    const uint16_t h = f2bf(v);
     wf[idx] = h;
     wb[((size_t)(TAPS - 1 - t) * C + k) * C + n] = h;
+}
+
+__global__ void kc_prep_weights(const float *__restrict__ W, uint16_t *__restrict__ wf, uint16_t *__restrict__ wb) {
+    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+    if (idx < TAPS * C * C) put_weight(idx, W[idx], wf, wb);
+}
+
+// The minibatch of step `step`: sample s of the batch is training pair
+// pick[step * batch + s]
+__global__ __launch_bounds__(256) void kc_pick(int V, int batch, int step, const int *__restrict__ pick,
+                                               const float *__restrict__ data_in, const float *__restrict__ data_t,
+                                               const float *__restrict__ data_tn, float *__restrict__ xin,
+                                               float *__restrict__ tgt, float *__restrict__ tn) {
+    const int s = blockIdx.y, p = pick[(size_t)step * batch + s];
+    const float *in = data_in + (size_t)p * V, *t = data_t + (size_t)p * V;
+    for (int v = blockIdx.x * 256 + threadIdx.x; v < V; v += gridDim.x * 256) {
+        xin[(size_t)s * V + v] = in[v];
+        tgt[(size_t)s * V + v] = t[v];
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) tn[s] = data_tn[p];
 }
 
 // round an FP32 tensor to bf16
@@ -724,11 +742,17 @@ __global__ __launch_bounds__(256) void kc_loss(int V, int B, int nblk, const flo
     if (threadIdx.x == 0) part[(size_t)s * nblk + blockIdx.x] = red[0];
 }
 
+// the bf16 weights of the layers, which the optimiser keeps up to date
+constexpr int MAX_LAYERS = 4;
+struct LayerWeights {
+    uint16_t *wf[MAX_LAYERS], *wb[MAX_LAYERS];
+};
+
 // Adam (Kingma and Ba, 2015) on FP32 master parameters; mask[i] == 0 keeps a
-// padded parameter at zero.
+// padded parameter at zero.  layer_len parameters per layer, weights first.
 __global__ void kc_adam(int n, float *__restrict__ p, const float *__restrict__ g, float *__restrict__ m,
                         float *__restrict__ v, const uint8_t *__restrict__ mask, float lr, float b1, float b2,
-                        float eps, float c1, float c2) {
+                        float eps, float c1, float c2, int layer_len, LayerWeights lw) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n || !mask[i]) return;
     const float gi = g[i];
@@ -736,7 +760,10 @@ __global__ void kc_adam(int n, float *__restrict__ p, const float *__restrict__ 
     const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    p[i] = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    const float pi = p[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
+    p[i] = pi;
+    const int l = i / layer_len, j = i % layer_len;
+    if (j < TAPS * C * C) put_weight(j, pi, lw.wf[l], lw.wb[l]);
 }
 
 }  // namespace cnn

@@ -28,6 +28,9 @@ constexpr int GAIN = NPARAM - 1;
 constexpr int WCHUNK = 4096;           // rows per partial weight and bias gradient
 constexpr int LOSS_BLK = 64;           // workgroups per sample in the loss
 
+// training steps whose losses stay on the device: at most 1024, 16 MB of partial sums
+int loss_steps(int max_batch) { return std::max(1, std::min(1024, (1 << 22) / LOSS_BLK / max_batch)); }
+
 thread_local std::string g_cnn_err;
 
 }  // namespace
@@ -43,6 +46,7 @@ struct plsqr_cnn {
     float *zout = nullptr, *dz1 = nullptr;  // output and its gradient, one channel
     uint16_t *dz[2] = {};             // gradients of the layers' outputs below
     float *wpart = nullptr, *bpart = nullptr, *lpart = nullptr;
+    int *pick = nullptr;  // training pairs of loss_steps(max_batch) steps
     float *xin = nullptr, *tgt = nullptr, *tn = nullptr, *x0 = nullptr;
     int count = 0;
     float *data_in = nullptr, *data_t = nullptr, *data_tn = nullptr;
@@ -222,23 +226,24 @@ int wgrad_first(plsqr_cnn *h, long long total, const uint16_t *dout, float *gw, 
     return PLSQR_OK;
 }
 
-// loss of zout against tgt/tn (batch samples), dz1 = its gradient; *loss on the host
-int loss_and_grad(plsqr_cnn *h, int batch, double *loss) {
+// loss of zout against tgt/tn (batch samples) as partial sums in lpart, dz1 =
+// its gradient
+int loss_and_grad(plsqr_cnn *h, int batch, float *lpart) {
     hipLaunchKernelGGL(kc_loss, dim3(LOSS_BLK, batch), dim3(256), 0, h->stream, h->V, batch, LOSS_BLK,
-                       (const float *)h->zout, (const float *)h->tgt, (const float *)h->tn, h->dz1, h->lpart);
+                       (const float *)h->zout, (const float *)h->tgt, (const float *)h->tn, h->dz1, lpart);
     CN_LAUNCH(h);
-    std::vector<float> part((size_t)batch * LOSS_BLK), tn((size_t)batch);
-    CN_TRY(h, hipMemcpyAsync(part.data(), h->lpart, sizeof(float) * part.size(), hipMemcpyDeviceToHost, h->stream));
-    CN_TRY(h, hipMemcpyAsync(tn.data(), h->tn, sizeof(float) * tn.size(), hipMemcpyDeviceToHost, h->stream));
-    CN_TRY(h, hipStreamSynchronize(h->stream));
+    return PLSQR_OK;
+}
+
+// the loss from its partial sums and the samples' target norms
+double loss_of(const float *part, const float *tn, int batch) {
     double L = 0.0;
     for (int s = 0; s < batch; ++s) {
         double e = 0.0;
         for (int b = 0; b < LOSS_BLK; ++b) e += part[(size_t)s * LOSS_BLK + b];
-        L += e / tn[(size_t)s];
+        L += e / tn[s];
     }
-    *loss = L / batch;
-    return PLSQR_OK;
+    return L / batch;
 }
 
 int backward(plsqr_cnn *h, int batch) {
@@ -408,7 +413,8 @@ int plsqr_cnn_create(int nx, int ny, int nz, int max_batch, unsigned long long s
         (rc = calloc_dev(h, &h->dz1, (size_t)total)) ||
         (rc = calloc_dev(h, &h->dz[0], (size_t)total * C)) || (rc = calloc_dev(h, &h->dz[1], (size_t)total * C)) ||
         (rc = calloc_dev(h, &h->wpart, (size_t)nch * TAPS * C * C)) || (rc = calloc_dev(h, &h->bpart, (size_t)nch * C)) ||
-        (rc = calloc_dev(h, &h->lpart, (size_t)max_batch * LOSS_BLK)) || (rc = calloc_dev(h, &h->xin, (size_t)total)) ||
+        (rc = calloc_dev(h, &h->lpart, (size_t)loss_steps(max_batch) * max_batch * LOSS_BLK)) ||
+        (rc = calloc_dev(h, &h->pick, (size_t)loss_steps(max_batch) * max_batch)) || (rc = calloc_dev(h, &h->xin, (size_t)total)) ||
         (rc = calloc_dev(h, &h->tgt, (size_t)total)) || (rc = calloc_dev(h, &h->tn, (size_t)max_batch)) ||
         (rc = calloc_dev(h, &h->x0, (size_t)total)))
         return fail(rc);
@@ -524,36 +530,55 @@ int plsqr_cnn_train(plsqr_cnn *h, int steps, int batch, float lr, unsigned long 
     Rng rng{seed};
     size_t pos = order.size();
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    for (int it = 0; it < steps; ++it) {
-        std::vector<int> pick((size_t)batch);
-        for (int s = 0; s < batch; ++s) {
+    LayerWeights lw;
+    static_assert(LAYERS <= MAX_LAYERS, "a pair of weight arrays per layer");
+    for (int l = 0; l < LAYERS; ++l) {
+        lw.wf[l] = h->wf[l];
+        lw.wb[l] = h->wb[l];
+    }
+    std::vector<int> pick;
+    std::vector<float> part, tn((size_t)h->count);
+    CN_TRY(h, hipMemcpyAsync(tn.data(), h->data_tn, sizeof(float) * tn.size(), hipMemcpyDeviceToHost, h->stream));
+    CN_TRY(h, hipStreamSynchronize(h->stream));
+    // the picks of many steps go to the device together and their losses come
+    // back together, so the steps are queued without waiting
+    const int group = loss_steps(h->max_batch);
+    for (int it0 = 0; it0 < steps; it0 += group) {
+        const int n = std::min(group, steps - it0);
+        pick.resize((size_t)n * batch);
+        for (int &p : pick) {
             if (pos >= order.size()) {  // a new epoch: Fisher-Yates shuffle
                 for (int i = 0; i < h->count; ++i) order[(size_t)i] = i;
                 for (int i = h->count - 1; i > 0; --i) std::swap(order[(size_t)i], order[(size_t)(rng.next() % (uint64_t)(i + 1))]);
                 pos = 0;
             }
-            pick[(size_t)s] = order[pos++];
+            p = order[pos++];
         }
-        for (int s = 0; s < batch; ++s) {
-            const size_t src = (size_t)pick[(size_t)s] * h->V;
-            CN_TRY(h, hipMemcpyAsync(h->xin + (size_t)s * h->V, h->data_in + src, sizeof(float) * h->V,
-                                     hipMemcpyDeviceToDevice, h->stream));
-            CN_TRY(h, hipMemcpyAsync(h->tgt + (size_t)s * h->V, h->data_t + src, sizeof(float) * h->V,
-                                     hipMemcpyDeviceToDevice, h->stream));
-            CN_TRY(h, hipMemcpyAsync(h->tn + s, h->data_tn + pick[(size_t)s], sizeof(float), hipMemcpyDeviceToDevice,
-                                     h->stream));
+        CN_TRY(h, hipMemcpyAsync(h->pick, pick.data(), sizeof(int) * pick.size(), hipMemcpyHostToDevice, h->stream));
+        for (int it = 0; it < n; ++it) {
+            hipLaunchKernelGGL(kc_pick, dim3(grid_for(h->V, 256, 64), batch), dim3(256), 0, h->stream, h->V, batch, it,
+                               (const int *)h->pick, (const float *)h->data_in, (const float *)h->data_t,
+                               (const float *)h->data_tn, h->xin, h->tgt, h->tn);
+            CN_LAUNCH(h);
+            if ((rc = forward(h, batch)) || (rc = loss_and_grad(h, batch, h->lpart + (size_t)it * batch * LOSS_BLK)) ||
+                (rc = backward(h, batch)))
+                return rc;
+            ++h->adam_t;
+            const float c1 = 1.f - std::pow(b1, (float)h->adam_t), c2 = 1.f - std::pow(b2, (float)h->adam_t);
+            hipLaunchKernelGGL(kc_adam, dim3((NPARAM + 255) / 256), dim3(256), 0, h->stream, NPARAM, h->params,
+                               (const float *)h->grads, h->adam_m, h->adam_v, (const uint8_t *)h->mask, lr, b1, b2, eps, c1,
+                               c2, LSZ, lw);
+            CN_LAUNCH(h);
         }
-        double loss;
-        if ((rc = forward(h, batch)) || (rc = loss_and_grad(h, batch, &loss)) || (rc = backward(h, batch))) return rc;
-        ++h->adam_t;
-        const float c1 = 1.f - std::pow(b1, (float)h->adam_t), c2 = 1.f - std::pow(b2, (float)h->adam_t);
-        hipLaunchKernelGGL(kc_adam, dim3((NPARAM + 255) / 256), dim3(256), 0, h->stream, NPARAM, h->params,
-                           (const float *)h->grads, h->adam_m, h->adam_v, (const uint8_t *)h->mask, lr, b1, b2, eps, c1, c2);
-        CN_LAUNCH(h);
-        h->weights_dirty = true;
-        if (loss_out) loss_out[it] = loss;
+        part.resize((size_t)n * batch * LOSS_BLK);
+        CN_TRY(h, hipMemcpyAsync(part.data(), h->lpart, sizeof(float) * part.size(), hipMemcpyDeviceToHost, h->stream));
+        CN_TRY(h, hipStreamSynchronize(h->stream));
+        std::vector<float> tb((size_t)batch);
+        for (int it = 0; loss_out && it < n; ++it) {
+            for (int s = 0; s < batch; ++s) tb[(size_t)s] = tn[(size_t)pick[(size_t)it * batch + s]];
+            loss_out[it0 + it] = loss_of(part.data() + (size_t)it * batch * LOSS_BLK, tb.data(), batch);
+        }
     }
-    CN_TRY(h, hipStreamSynchronize(h->stream));
     return PLSQR_OK;
 }
 
@@ -563,9 +588,13 @@ int plsqr_cnn_gradient(plsqr_cnn *h, int batch, const double *atb, const double 
     if (batch < 1 || batch > h->max_batch || !atb || !xstar || !grads || !loss)
         return set_err(h, PLSQR_ERR_ARG, "bad gradient arguments");
     if ((rc = load_samples(h, batch, atb, xstar, nullptr))) return rc;
-    if ((rc = forward(h, batch)) || (rc = loss_and_grad(h, batch, loss)) || (rc = backward(h, batch))) return rc;
+    if ((rc = forward(h, batch)) || (rc = loss_and_grad(h, batch, h->lpart)) || (rc = backward(h, batch))) return rc;
+    std::vector<float> part((size_t)batch * LOSS_BLK), tn((size_t)batch);
+    CN_TRY(h, hipMemcpyAsync(part.data(), h->lpart, sizeof(float) * part.size(), hipMemcpyDeviceToHost, h->stream));
+    CN_TRY(h, hipMemcpyAsync(tn.data(), h->tn, sizeof(float) * tn.size(), hipMemcpyDeviceToHost, h->stream));
     CN_TRY(h, hipMemcpyAsync(grads, h->grads, sizeof(float) * NPARAM, hipMemcpyDeviceToHost, h->stream));
     CN_TRY(h, hipStreamSynchronize(h->stream));
+    *loss = loss_of(part.data(), tn.data(), batch);
     return PLSQR_OK;
 }
 
