@@ -1325,14 +1325,25 @@ static void launch_cols_tiled32(plsqr_op *op, const float *u, const Scal *sc) {
                        op->tS, op->t_start, op->t_slot, op->t_seg, op->t_vlen, op->t_ray, op->t_sval32, op->t_sseg,   \
                        op->t_cut, op->t_vcut, sr, u, sc, op->P);
     // 512 threads (two per voxel) on 256-voxel tiles: 36 KB of LDS, so four
-    // items share a CU and one item's staging overlaps the others' slot loops
+    // items share a CU and one item's staging overlaps the others' slot loops.
+    // With fewer than two rounds of those (8 items per CU), 1024 threads: an
+    // item takes half as long and the CUs fill as well (mode 2 in us, 512 / 1024
+    // threads: 24^3 864 items 24.0 / 17.4, 32^3 1024 items 36.2 / 30.5, 37 x 29 x
+    // 41 1376 items 44.4 / 42.2; 48^3 3456 items 104.6 / 107.0, 67^3 344 / 356).
+    const bool few = op->tT * op->tS <= 8 * op->cu;
+#define COLS32_256(FORM)                \
+    if (few) {                          \
+        COLS32(256, 1024, 8192, FORM)   \
+    } else {                            \
+        COLS32(256, 512, 8192, FORM)    \
+    }
     if (op->tw == 256) {
         if (op->t_form == 1) {
-            COLS32(256, 512, 8192, 1)
+            COLS32_256(1)
         } else if (op->t_form == 2) {
-            COLS32(256, 512, 8192, 2)
+            COLS32_256(2)
         } else {
-            COLS32(256, 512, 8192, 0)
+            COLS32_256(0)
         }
     } else if (op->t_form == 1) {
         COLS32(TILE_W, 512, 4096, 1)
@@ -1341,6 +1352,7 @@ static void launch_cols_tiled32(plsqr_op *op, const float *u, const Scal *sc) {
     } else {
         COLS32(TILE_W, 512, 4096, 0)
     }
+#undef COLS32_256
 #undef COLS32
 }
 
