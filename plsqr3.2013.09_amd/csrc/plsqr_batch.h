@@ -276,19 +276,14 @@ __global__ __launch_bounds__(BS) void kb_seg(const int *__restrict__ blk_item, c
     for (int i = threadIdx.x; i < tw * K; i += BS) xl[i] = x[(size_t)c0 * K + i];
     __syncthreads();
     const int lane = threadIdx.x % G;
-    const int wv = threadIdx.x / G;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / G);
     T *bv = lv[wv];
     uint8_t *bx = lx[wv];
     const long long sb = seg_start[it];
     for (int g = g0 + wv; g < g1; g += NWV) {
         const int len = seg_len[(size_t)g * G + lane];
-        int incl = len;
-#pragma unroll
-        for (int o = 1; o < G; o <<= 1) {
-            const int up = __shfl_up(incl, o);
-            if (lane >= o) incl += up;
-        }
-        const int tot = __shfl(incl, G - 1);
+        const int incl = wave_prefix_sum(len);
+        const int tot = __builtin_amdgcn_readlane(incl, G - 1);
         const int beg = incl - len, end = incl;
         const long long gb = ent_base[g];
         Acc<T> acc[K];

@@ -111,7 +111,7 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_c32(int S, const int *__restr
     for (int i = threadIdx.x; i < tw; i += BS) xl[i] = (double)x[c0 + i];
     __syncthreads();
     const int lane = threadIdx.x % G;
-    const int wv = threadIdx.x / G;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / G);
     float *bv = lv[wv];
     uint8_t *bx = lx[wv];
     const long long sb = seg_start[it];
@@ -131,13 +131,8 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_c32(int S, const int *__restr
         } else if constexpr (TW > 256) {
             h1 = seg_lo[(size_t)g * G + lane];
         }
-        int incl = len;
-#pragma unroll
-        for (int o = 1; o < G; o <<= 1) {
-            const int up = __shfl_up(incl, o);
-            if (lane >= o) incl += up;
-        }
-        const int tot = __shfl(incl, G - 1);
+        const int incl = wave_prefix_sum(len);
+        const int tot = __builtin_amdgcn_readlane(incl, G - 1);
         const int beg = incl - len, end = incl;
         h1 += beg;
         h2 += beg;

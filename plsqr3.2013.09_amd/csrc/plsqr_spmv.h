@@ -164,7 +164,7 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_c(int S, const int *__restric
     for (int i = threadIdx.x; i < tw; i += BS) xl[i] = x[c0 + i];
     __syncthreads();
     const int lane = threadIdx.x % G;
-    const int wv = threadIdx.x / G;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / G);
     double *bv = lv[wv];
     uint8_t *bx = lx[wv];
     const long long sb = seg_start[it];
@@ -184,13 +184,8 @@ __global__ __launch_bounds__(BS) void k_rows_tiled_c(int S, const int *__restric
         } else if constexpr (TW > 256) {
             h1 = seg_lo[(size_t)g * G + lane];
         }
-        int incl = len;
-#pragma unroll
-        for (int o = 1; o < G; o <<= 1) {
-            const int up = __shfl_up(incl, o);
-            if (lane >= o) incl += up;
-        }
-        const int tot = __shfl(incl, G - 1);  // entries of the group
+        const int incl = wave_prefix_sum(len);
+        const int tot = __builtin_amdgcn_readlane(incl, G - 1);  // entries of the group
         const int beg = incl - len, end = incl;
         h1 += beg;
         h2 += beg;
