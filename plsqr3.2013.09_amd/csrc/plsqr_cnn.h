@@ -526,39 +526,45 @@ __global__ __launch_bounds__(256, 2) void kc_wgrad(int nx, int ny, int nz, long 
     }
 }
 
-// p[0] + p[stride] + .. (count terms, in order), sixteen loads in flight
+// p[0] + p[stride] + .. (count terms, in order), FLIGHT loads in flight: the
+// last repeated past the end and not added
+template <int FLIGHT>
 __device__ __forceinline__ float ordered_sum(const float *__restrict__ p, int count, size_t stride) {
     float s = 0.f;
-    int c = 0;
-    for (; c + 16 <= count; c += 16) {
-        float v[16];
+    for (int c = 0; c < count; c += FLIGHT) {
+        float v[FLIGHT];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) v[k] = p[(size_t)(c + k) * stride];
+        for (int k = 0; k < FLIGHT; ++k) v[k] = p[(size_t)min(c + k, count - 1) * stride];
 #pragma unroll
-        for (int k = 0; k < 16; ++k) s += v[k];
+        for (int k = 0; k < FLIGHT; ++k)
+            if (c + k < count) s += v[k];
     }
-    for (; c < count; ++c) s += p[(size_t)c * stride];
     return s;
 }
 
 // Sums over chunks in order.  Weights: grad[t][n][k] of part[t][chunk][n][k],
 // or with FIRST the one channel's grad[t][n][0] of part[chunk][n][t].  Bias
-// (the last workgroup): bgrad[n] of bpart[chunk][n].  The loads of sixteen
-// chunks are in flight together, so the serial sums wait for memory once in
-// sixteen (67^3 x 4: 294 chunks, weights 71 -> 15 us, bias 67 us before).
+// (the last workgroup): bgrad[n] of bpart[chunk][n].  Each sum is serial and
+// there are few of them (27 x 1024), so the loads in flight set the time: 48
+// per thread, in one-wavefront workgroups that reach all CUs (67^3 x 4: 294
+// chunks, 16.3 -> 9.4 us; 16 per thread in 256-thread workgroups before,
+// 71 us with one).
+constexpr int GRAD_RED = 64;  // threads per workgroup
+
 template <bool FIRST>
-__global__ __launch_bounds__(256) void kc_grad_reduce(int nchunk, const float *__restrict__ part,
-                                                      const float *__restrict__ bpart, float *__restrict__ grad,
-                                                      float *__restrict__ bgrad) {
-    const int idx = blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(GRAD_RED) void kc_grad_reduce(int nchunk, const float *__restrict__ part,
+                                                           const float *__restrict__ bpart, float *__restrict__ grad,
+                                                           float *__restrict__ bgrad) {
+    constexpr int F = 48;
+    const int idx = blockIdx.x * GRAD_RED + threadIdx.x;
     if (blockIdx.x == gridDim.x - 1) {
-        if (threadIdx.x < C) bgrad[threadIdx.x] = ordered_sum(bpart + threadIdx.x, nchunk, C);
+        if (threadIdx.x < C) bgrad[threadIdx.x] = ordered_sum<F>(bpart + threadIdx.x, nchunk, C);
     } else if constexpr (FIRST) {
         const int n = idx / C, t = idx % C;
-        if (n < C && t < TAPS) grad[(t * C + n) * C] = ordered_sum(part + idx, nchunk, C * C);
+        if (n < C && t < TAPS) grad[(t * C + n) * C] = ordered_sum<F>(part + idx, nchunk, C * C);
     } else {
         const int t = idx / (C * C), e = idx % (C * C);
-        if (t < TAPS) grad[idx] = ordered_sum(part + (size_t)t * nchunk * (C * C) + e, nchunk, C * C);
+        if (t < TAPS) grad[idx] = ordered_sum<F>(part + (size_t)t * nchunk * (C * C) + e, nchunk, C * C);
     }
 }
 

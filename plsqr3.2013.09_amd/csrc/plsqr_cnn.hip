@@ -245,7 +245,7 @@ int wgrad(plsqr_cnn *h, int nx, int ny, int nz, long long total, const uint16_t 
     else
         hipLaunchKernelGGL((kc_wgrad<3, DONE>), dim3(blocks), dim3(256), 0, st, nx, ny, nz, total, WCHUNK, in, dout, wpart,
                            bpart);
-    hipLaunchKernelGGL((kc_grad_reduce<false>), dim3(WSZ / 256 + 1), dim3(256), 0, st, nch, (const float *)wpart,
+    hipLaunchKernelGGL((kc_grad_reduce<false>), dim3(WSZ / GRAD_RED + 1), dim3(GRAD_RED), 0, st, nch, (const float *)wpart,
                        (const float *)bpart, gw, gb);
     return hipGetLastError() == hipSuccess ? PLSQR_OK : set_err(h, PLSQR_ERR_HIP, "gradient kernels failed to launch");
 }
@@ -255,7 +255,7 @@ int wgrad_first(plsqr_cnn *h, long long total, const uint16_t *dout, float *gw, 
     const int nch = (int)((total + WCHUNK - 1) / WCHUNK);
     hipLaunchKernelGGL(kc_wgrad_first, dim3(nch), dim3(256), 0, h->stream, h->nx, h->ny, h->nz, total, WCHUNK,
                        (const float *)h->xin, dout, h->wpart, h->bpart);
-    hipLaunchKernelGGL((kc_grad_reduce<true>), dim3(C * C / 256 + 1), dim3(256), 0, h->stream, nch,
+    hipLaunchKernelGGL((kc_grad_reduce<true>), dim3(C * C / GRAD_RED + 1), dim3(GRAD_RED), 0, h->stream, nch,
                        (const float *)h->wpart, (const float *)h->bpart, gw, gb);
     CN_LAUNCH(h);
     return PLSQR_OK;
