@@ -564,6 +564,13 @@ int b_internal(plsqr_op *op, const double *b, const double **out) {
     return PLSQR_OK;
 }
 
+// Rows up to which mode 1 updates a caller-order y in place.  The combine's
+// scattered 8 or 4 bytes per row cost more than two reordering passes once y is
+// far larger than the L2s (FP64 / FP32 mode 1 in us, in place against reordered:
+// 0.52M rows 60 / 43 against 71 / 52, 1.1M 148 / 94 against 158 / 105, 2.2M
+// 403 / 259 against 404 / 264, 3.2M 553 / 364 against 550 / 360).
+constexpr int IN_PLACE_ROWS = 2500000;
+
 // aprod on operands each either in the caller's order (renumbered in and,
 // for the output, back) or already in the device order.  The tiled operator's
 // combines update a caller-order output in place.
@@ -571,7 +578,7 @@ int aprod_any(plsqr_op *op, int mode, double *x, bool x_ext, double *y, bool y_e
     int rc;
     const bool tiled = mode == 1 ? op->rtiled : op->tiled;
     const bool move_x = x_ext && op->permuted, move_y = y_ext && op->rowperm;
-    const bool place_x = mode == 2 && tiled && move_x, place_y = mode == 1 && tiled && move_y;
+    const bool place_x = mode == 2 && tiled && move_x, place_y = mode == 1 && tiled && move_y && op->m <= IN_PLACE_ROWS;
     double *xi = x, *yi = y;
     if (move_x && !place_x) {
         if ((rc = to_internal(op, x, op->hx2))) return rc;
@@ -1431,7 +1438,7 @@ int plsqr_aprod_device_f32(plsqr_op *op, int mode, float *x_dev, float *y_dev) {
     if ((rc = ensure_aprod32(op))) return rc;
     const int gn = grid_for(op->n, 256, op->cu * 4), gm = grid_for(op->m, 256, op->cu * 4);
     // caller order -> device order, except an output that a combine updates in place
-    const bool place_x = mode == 2 && op->permuted, place_y = mode == 1 && op->rowperm && op->rtiled;
+    const bool place_x = mode == 2 && op->permuted, place_y = mode == 1 && op->rowperm && op->rtiled && op->m <= IN_PLACE_ROWS;
     if (!place_x) {
         if (op->permuted)
             hipLaunchKernelGGL(k_gather32, dim3(gn), dim3(256), 0, op->stream, op->n, op->inv, x_dev, op->v32);
