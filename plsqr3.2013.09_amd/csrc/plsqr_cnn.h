@@ -329,6 +329,165 @@ __global__ __launch_bounds__(CONV_THREADS, 2) void kc_conv(int nx, int ny, int n
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same layer for grids that fill bricks badly: a wavefront takes 32
+// consecutive rows whatever their place in the grid, so thin and tiny grids cost
+// no matrix steps for voxels that do not exist.  All weights lie in LDS; for one
+// dz at a time the wavefront's three runs of 34 consecutive rows (dy -1, 0, 1)
+// pass through LDS as bf16, the loads of the next dz in flight while this one is
+// multiplied.  What bounds it is staging each row nine times; fragments loaded
+// straight from memory, 32 cache lines per load, were bound by the L1 (131072
+// voxels, FP32: 69 us, here 23).  A tap without a neighbour multiplies zeros.
+// Taps and K steps are added in kc_conv's order, so both give the same bits.
+// 120 KB of LDS: one workgroup per CU stays for all of its rows.
+// ---------------------------------------------------------------------------
+template <int IN, bool WF32, int OUT>
+__global__ __launch_bounds__(CONV_THREADS, 2) void kc_conv_rows(int nx, int ny, int nz, unsigned total, const void *__restrict__ in,
+                                                                const void *__restrict__ w, const float *__restrict__ bias,
+                                                                const uint16_t *__restrict__ mask, int relu,
+                                                                void *__restrict__ out, int aligned) {
+    constexpr int KS = IN == CONV_ONE ? 1 : 2;
+    constexpr int RUN = 34;                                            // rows of a run
+    constexpr int PIECES = IN == CONV_F32 ? 8 : IN == CONV_BF16 ? 4 : 1;  // loads per row: four floats, eight bf16 or one float
+    constexpr int PER = (RUN * PIECES + 63) / 64;
+    constexpr int VS = IN == CONV_ONE ? 1 : 5;                         // 16-byte units per row in LDS (4 of data)
+    __shared__ uint4_t wl[TAPS * KS * 64];
+    __shared__ uint4_t xs[CB][3][RUN * VS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = lane & 31, h = lane >> 5;
+    // weight fragments as in kc_conv
+    const bool wide = ((uintptr_t)w & 15) == 0;
+#pragma unroll
+    for (int j = 0; j < (TAPS * KS * 64 + CONV_THREADS - 1) / CONV_THREADS; ++j) {
+        const int f = threadIdx.x + j * CONV_THREADS;
+        if (f >= TAPS * KS * 64) break;
+        const int src = ((f >> 6) / KS * C + (f & 31)) * C + 16 * ((f >> 6) % KS) + 8 * (f >> 5 & 1);
+        if constexpr (!WF32) {
+            wl[f] = *(const uint4_t *)((const uint16_t *)w + src);
+        } else {
+            const float *p = (const float *)w + src;
+            float4 a, b;
+            if (wide)
+                a = ((const float4 *)p)[0], b = ((const float4 *)p)[1];
+            else
+                a = make_float4(p[0], p[1], p[2], p[3]), b = make_float4(p[4], p[5], p[6], p[7]);
+            wl[f] = uint4_t{pack_bf(a.x, a.y), pack_bf(a.z, a.w), pack_bf(b.x, b.y), pack_bf(b.z, b.w)};
+        }
+    }
+    float bn[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) bn[r] = bias ? bias[8 * (r / 4) + 4 * h + r % 4] : 0.f;
+    __syncthreads();
+    const unsigned groups = (total + 31) / 32;
+    for (unsigned gr = blockIdx.x * CB + wave; gr < groups; gr += gridDim.x * CB) {
+        const unsigned g = min(gr * 32 + i, total - 1);  // past the end: the last row again, not stored
+        const unsigned line = g / (unsigned)nx, plane = line / (unsigned)ny;
+        const int x = (int)(g - line * nx), y = (int)(line - plane * ny), z = (int)(plane % (unsigned)nz);
+        uint2_t mk[4];
+        if constexpr (OUT == CONV_BF16) {
+            if (mask) {
+#pragma unroll
+                for (int b = 0; b < 4; ++b) mk[b] = *(const uint2_t *)(mask + (size_t)g * C + 8 * b + 4 * h);
+            }
+        }
+        uint4_t u[3][PER];
+        auto load = [&](int dz) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) {
+                const long long first = (long long)gr * 32 - 1 + ((long long)dz * ny + q - 1) * nx;
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    const int p = min(lane + 64 * j, RUN * PIECES - 1);
+                    // rows outside the tensor are no row's neighbour
+                    const long long r = min(max(first + p / PIECES, 0LL), (long long)total - 1);
+                    const long long src = r * PIECES + p % PIECES;
+                    if constexpr (IN == CONV_ONE) {
+                        u[q][j][0] = ((const uint32_t *)in)[src];
+                    } else if (IN == CONV_BF16 || aligned) {
+                        u[q][j] = ((const uint4_t *)in)[src];
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) u[q][j][e] = ((const uint32_t *)in)[src * 4 + e];
+                    }
+                }
+            }
+        };
+        auto store = [&]() {
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+#pragma unroll
+                for (int j = 0; j < PER; ++j) {
+                    const int p = lane + 64 * j, row = p / PIECES, c = p % PIECES;
+                    if (p >= RUN * PIECES) break;
+                    uint4_t *const to = xs[wave][q] + row * VS;
+                    if constexpr (IN == CONV_ONE)
+                        to[0] = uint4_t{f2bf(__uint_as_float(u[q][j][0])), 0, 0, 0};
+                    else if constexpr (IN == CONV_BF16)
+                        to[c] = u[q][j];
+                    else
+                        ((uint2_t *)to)[c] = uint2_t{pack_bf(__uint_as_float(u[q][j][0]), __uint_as_float(u[q][j][1])),
+                                                     pack_bf(__uint_as_float(u[q][j][2]), __uint_as_float(u[q][j][3]))};
+                }
+        };
+        floatx16 acc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+        load(-1);
+#pragma unroll 1
+        for (int dz = -1; dz <= 1; ++dz) {
+            store();
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (dz < 1) load(dz + 1);
+            const uint4_t *const wt = wl + (dz + 1) * 9 * KS * 64 + lane;
+#pragma unroll
+            for (int t = 0; t < 9; ++t) {
+                const int q = t / 3, dx = t % 3 - 1;
+                const bool ok = (unsigned)(z + dz) < (unsigned)nz && (unsigned)(y + q - 1) < (unsigned)ny && (unsigned)(x + dx) < (unsigned)nx;
+#pragma unroll
+                for (int s = 0; s < KS; ++s) {
+                    uint4_t b = xs[wave][q][(i + t % 3) * VS + (IN == CONV_ONE ? 0 : 2 * s + h)];
+                    if (!ok || (IN == CONV_ONE && h == 1)) b = uint4_t{0, 0, 0, 0};
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wt[(t * KS + s) * 64]),
+                                                                  __builtin_bit_cast(bf16x8, b), acc, 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+        if (gr * 32 + i >= total) continue;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            const size_t o = (size_t)g * C + 8 * b + 4 * h;  // channels 8b + 4h .. +3
+            float v[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                v[k] = acc[4 * b + k] + bn[4 * b + k];
+                if (relu) v[k] = fmaxf(v[k], 0.f);
+            }
+            if constexpr (OUT == CONV_BF16) {
+                if (mask) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k)
+                        if (!(bf2f((uint16_t)(mk[b][k / 2] >> (16 * (k % 2)))) > 0.f)) v[k] = 0.f;
+                }
+                *(uint2_t *)((uint16_t *)out + o) = uint2_t{pack_bf(v[0], v[1]), pack_bf(v[2], v[3])};
+            } else if constexpr (OUT == CONV_ONE) {
+                if (b == 0 && h == 0) ((float *)out)[g] = v[0];
+            } else {
+                float *d = (float *)out + o;
+                if (aligned) {
+                    *(float4 *)d = make_float4(v[0], v[1], v[2], v[3]);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) d[k] = v[k];
+                }
+            }
+        }
+    }
+}
+
 // s + this thread's rows q, q + 8, .. of the first `live` rows of staged dout
 // (a multiple of 64 rows is readable), thread (q, n) = (tid / 32, tid % 32)
 __device__ __forceinline__ float bias_rows(float s, const uint16_t *rows, int live) {

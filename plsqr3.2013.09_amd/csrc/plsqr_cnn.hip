@@ -194,17 +194,31 @@ int compute_units() {
     return cu;
 }
 
-// One convolution layer over `samples` grids (kc_conv): one workgroup per CU,
-// or per brick where there are fewer; a multiple of eight when it can be, so
-// that each XCD takes one range of bricks.
+// One convolution layer over `samples` grids.  By bricks (kc_conv): one workgroup
+// per CU, or per brick where there are fewer; a multiple of eight when it can be,
+// so that each XCD takes one range of bricks.  By rows (kc_conv_rows) where that
+// takes fewer than half as many rounds over the CUs, a round being a brick or 256
+// rows per CU: a round of bricks takes 3 to 8 us however few voxels they hold.
+// FP32 layers in us, rounds and times by bricks against by rows: 131072 grids of
+// one voxel 512 / 2, 1465 / 23; 1 x 1 x 131072 64 / 2, 262 / 23; 256 grids of
+// 1 x 16 x 16 4 / 1, 31 / 14; 170 of 9^3 6 / 2, 51 / 22; 69 of 25 x 25 x 3 5 / 2,
+// 31 / 26.  Below the line: 1024 of 5 x 4 x 4 4 / 2, 19.5 / 20.8; 512 of 3^3 2 / 1,
+// 12.0 / 12.6; 200 x 2 x 200 3 / 2, 21 / 24; 32 of 16^3 1 / 2, 18 / 24.
 template <int IN, bool WF32, int OUT>
 void conv(int nx, int ny, int nz, int samples, const void *in, const void *w, const float *bias, const uint16_t *mask,
           int relu, void *out, hipStream_t st) {
     auto bricks = [](int n) { return (long long)((n + CB - 1) / CB); };
-    const long long tiles = bricks(nx) * bricks(ny) * bricks(nz) * samples;
-    long long g = std::min<long long>(tiles, compute_units());
+    const long long tiles = bricks(nx) * bricks(ny) * bricks(nz) * samples, rows = (long long)nx * ny * nz * samples;
+    const int aligned = (((uintptr_t)in | (uintptr_t)out) & 15) == 0, cus = compute_units();
+    const long long brick_rounds = (tiles + cus - 1) / cus, row_blocks = (rows + 32 * CB - 1) / (32 * CB);
+    if (brick_rounds > 2 * ((row_blocks + cus - 1) / cus)) {
+        const long long g = std::min<long long>(row_blocks, cus);
+        hipLaunchKernelGGL((kc_conv_rows<IN, WF32, OUT>), dim3((unsigned)g), dim3(CONV_THREADS), 0, st, nx, ny, nz, (unsigned)rows,
+                           in, w, bias, mask, relu, out, aligned);
+        return;
+    }
+    long long g = std::min<long long>(tiles, cus);
     if (g >= 8) g = g / 8 * 8;
-    const int aligned = (((uintptr_t)in | (uintptr_t)out) & 15) == 0;
     hipLaunchKernelGGL((kc_conv<IN, WF32, OUT>), dim3((unsigned)g), dim3(CONV_THREADS), 0, st, nx, ny, nz, samples, in, w,
                        bias, mask, relu, out, aligned);
 }
