@@ -254,7 +254,8 @@ int forward(plsqr_cnn *h, int batch) {
     return PLSQR_OK;
 }
 
-// Weight and bias gradients of one layer; DONE: dout is one channel (FP32).
+// Weight and bias gradients of one layer; DONE: dout is one channel (FP32).  An
+// error is left with h, or without a handle for plsqr_cnn_last_error(NULL).
 template <bool DONE>
 int wgrad(plsqr_cnn *h, int nx, int ny, int nz, long long total, const uint16_t *in, const void *dout, float *gw,
           float *gb, float *wpart, float *bpart, hipStream_t st) {
@@ -746,8 +747,6 @@ int plsqr_cnn_conv_backward(int nx, int ny, int nz, int batch, const float *in, 
     if (nx < 1 || ny < 1 || nz < 1 || batch < 1 || !in || !w || !dout || !din || !dw || !dbias)
         return set_err(nullptr, PLSQR_ERR_ARG, "bad arguments");
     const long long total = (long long)batch * nx * ny * nz;
-    plsqr_cnn tmp;
-    plsqr_cnn *h = &tmp;
     const int nch = (int)((total + WCHUNK - 1) / WCHUNK);
     float *fin = nullptr, *fw = nullptr, *fdo = nullptr, *fdi = nullptr, *gw = nullptr, *wpart = nullptr, *bpart = nullptr;
     uint16_t *bin = nullptr, *bdo = nullptr, *wf = nullptr, *wb = nullptr;
@@ -774,7 +773,7 @@ int plsqr_cnn_conv_backward(int nx, int ny, int nz, int batch, const float *in, 
         hipLaunchKernelGGL(kc_to_bf16, dim3(g), dim3(256), 0, 0, total * C, (const float *)fdo, bdo);
         hipLaunchKernelGGL(kc_prep_weights, dim3((WSZ + 255) / 256), dim3(256), 0, 0, (const float *)fw, wf, wb);
         conv<CONV_BF16, false, CONV_F32>(nx, ny, nz, batch, bdo, wb, nullptr, nullptr, 0, fdi, 0);
-        rc = wgrad<false>(h, nx, ny, nz, total, bin, bdo, gw, gw + WSZ, wpart, bpart, 0);
+        rc = wgrad<false>(nullptr, nx, ny, nz, total, bin, bdo, gw, gw + WSZ, wpart, bpart, 0);
         e = hipGetLastError();
         if (e == hipSuccess) e = hipDeviceSynchronize();
         if (e == hipSuccess) e = hipMemcpy(din, fdi, sizeof(float) * total * C, hipMemcpyDeviceToHost);

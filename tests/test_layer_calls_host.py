@@ -1,5 +1,6 @@
 """Host code of the layer calls on host arrays, run without a GPU on a stand-in
-for the HIP calls they make (native/hip_stub.c): how they allocate."""
+for the HIP calls they make (native/hip_stub.c): how they allocate, and what they
+report when a launch fails."""
 import os
 import shutil
 import subprocess
@@ -53,3 +54,9 @@ def test_small_buffers_stay_on_the_fast_allocations(tmp_path, call, grid, most):
         assert max(sizes) < 2 << 20
     else:
         assert len(sizes) == 1
+
+
+@pytest.mark.parametrize("call", ["forward", "backward"])
+def test_a_failed_launch_is_reported_with_its_message(tmp_path, call):
+    last, _ = layer_call(tmp_path, call, "5x4x3", launch=1)
+    assert last.startswith("error 4 plsqr error HIP: ") and last != "error 4 plsqr error HIP: ", last
