@@ -491,8 +491,8 @@ void default_opts(const plsqr_solve_opts *o, plsqr_solve_opts *d) {
     if (d->refine_every <= 0) d->refine_every = 25;
 }
 
-// runs `count` graph launches, polling the live count every 8; returns the
-// number launched.  Records b->evs[first + i] after launch i.
+// runs `count` graph launches, with a tolerance polling the live count every 8;
+// returns the number launched.  Records b->evs[first + i] after launch i.
 // ratio_d (may be NULL): per state the FP64 / inner test2 ratio of the last
 // check; with it the chunk also ends once a live state's predicted test2
 // reaches tol, but not before min_pred launches: a check costs the whole
@@ -508,9 +508,10 @@ int run_launches(plsqr_batch *b, hipGraphExec_t exec, int count, size_t first, i
         BT_TRY(b, hipEventRecord(b->evs[first + (size_t)i], b->stream));
         ++*launched;
         // without a tolerance only states that never start (b = 0) end early, so
-        // one poll finds them; each poll drains the queue (6 grids of 12^3..24^3:
-        // 3 us of 207 per iteration)
-        if ((i + 1) % 8 == 0 && i + 1 < count && (tol > 0.0 || i + 1 == 8)) {
+        // one poll finds them, after the first launch (grids of 40^3 and 30^3, four
+        // right-hand sides, all zero: 112 us, after the eighth 333); each poll drains
+        // the queue (6 grids of 12^3..24^3: 3 us of 207 per iteration)
+        if (tol > 0.0 ? (i + 1) % 8 == 0 && i + 1 < count : i == 0 && count > 8) {
             if (ratio_d)
                 hipLaunchKernelGGL(kb_count_pred, dim3(1), dim3(256), 0, b->stream, b->P * b->K, (const Scal *)b->sc,
                                    ratio_d, tol, b->live_d);
