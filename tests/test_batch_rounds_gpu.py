@@ -1,8 +1,46 @@
-"""Batches at the ends of their iteration loop: right-hand sides that are all zero."""
+"""Batches where their loops end otherwise than in the common case: items with
+more segments than mode 2 stages in LDS at once, and right-hand sides that are
+all zero.
+
+Tolerance of the products: sums of up to 50,000 terms in another order stay
+within 2^-53 sqrt(50000) = 2.5e-14 of the result's norm in FP64, 1e-13 asked;
+FP32 operands and results with FP64 sums round to a few 2^-24, 1e-6 asked.
+"""
 import numpy as np
 import pytest
 
+from conftest import rel
+
 pytestmark = pytest.mark.gpu
+
+MAX_SLICES = 64  # of a problem's rows
+# every launch shape of mode 2
+SHAPES2 = [dict(rows_per_wave=4, nnz_per_lane=4, block_rows=256, block_cols=c, gather_kib=k)
+           for c in (128, 256, 512) for k in (32, 64)]
+
+
+@pytest.mark.parametrize("rhs,rays", [(1, 1100000), (2, 550000), (3, 300000), (4, 300000)])
+def test_mode2_in_rounds_matches_oracle(P, O, gpu_available, rhs, rays):
+    """All rays cross the one brick, so an item of at most 64 slices has
+    rays / 64 segments on average, more than the largest staging capacity."""
+    print(f"batch rounds: {rays} rays through one brick, {rhs} right-hand sides", flush=True)
+    s = P.generate(4, 4, 8, rays, P.GEOM_OPPOSITE_FACES, 3, 0.02, 0.1)
+    assert np.unique(s.k_row_idx).size == rays
+    width = 4 if rhs == 3 else rhs
+    assert rays / MAX_SLICES > 64 * 1024 // (4 * width), "FP32 in 64 KiB holds the most segments"
+    orc = O.Oracle(s)
+    rng = np.random.default_rng(rhs)
+    X, Y = rng.standard_normal((rhs, s.n)), rng.standard_normal((rhs, s.m_k + s.m_d))
+    want = X.copy()
+    for k in range(rhs):
+        orc.aprod(2, want[k], Y[k].copy())
+    with P.Batch([s], rhs, flags=P.BATCH_NO_TUNE) as bt:
+        for shape in SHAPES2:
+            for precision, bar in ((P.PREC_FP64, 1e-13), (P.PREC_MIXED, 1e-6)):
+                bt.set_tuning(precision, **shape)
+                xg, _ = bt.aprod(2, [X.copy()], [Y], precision)
+                for k in range(rhs):
+                    assert rel(xg[0][k], want[k]) < bar, (shape, precision, k, rel(xg[0][k], want[k]))
 
 
 @pytest.mark.parametrize("itn", [8, 9, 400])
