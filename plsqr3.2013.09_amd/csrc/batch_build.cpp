@@ -207,7 +207,8 @@ int build_batch_plan(const plsqr_system *const *systems, const plsqr_grid *grids
         const int T = (int)tiles.size() - 1;
         const long long by_rows = (s->m_k + std::max(slice_rows, 1) - 1) / std::max(slice_rows, 1);
         const long long by_nnz = s->nnz_k / (T * item_nnz);
-        const int S = (int)std::max(1LL, std::min({64LL, std::max(by_rows, by_nnz), (long long)s->m_k}));
+        // (never more slices than rows: a tile has 128 columns, an item 1024 nonzeros or more)
+        const int S = (int)std::max(1LL, std::min(64LL, std::max(by_rows, by_nnz)));
         auto cut_slices = [S](const plsqr_system *q_s) {
             std::vector<int> sl((size_t)S + 1, 0);
             std::vector<long long> cnt((size_t)q_s->m_k + 1, 0);

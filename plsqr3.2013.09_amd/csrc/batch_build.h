@@ -73,8 +73,9 @@ int validate_system(const plsqr_system *s, std::string *err);
 
 // Builds the plan.  grids[p] may describe problem p's voxel grid (brick tiles
 // of 4 x 4 x 8) or be zero-sized / absent (tiles of TW consecutive columns).
-// Kernel rows are cut into slices of at most about slice_rows rows and of
-// about 4096 nonzeros (fewer in small batches) per tile (balanced by nonzeros); xcds is the number of L2 domains to queue the slices on.
+// Kernel rows are cut into at most 64 slices, balanced by nonzeros: of at most
+// about slice_rows rows and about 4096 nonzeros per tile (fewer in small
+// batches).  xcds is the number of L2 domains to queue the slices on.
 int build_batch_plan(const plsqr_system *const *systems, const plsqr_grid *grids, int P, int TW,
                      int row_chunk, int damp_chunk, int col_chunk, int slice_rows, int xcds, BatchPlan *plan,
                      std::string *err);
