@@ -47,20 +47,6 @@ __device__ __forceinline__ uint16_t f2bf(float f) { return __builtin_bit_cast(ui
 
 __device__ __forceinline__ float bf2f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
-// voxel coordinates of the flattened (sample, voxel) index g
-struct Vox {
-    int x, y, z;
-};
-
-__device__ __forceinline__ Vox vox_of(long long g, int nx, int ny, int V) {
-    const int v = (int)(g % V);
-    Vox r;
-    r.x = v % nx;
-    r.y = (v / nx) % ny;
-    r.z = v / (nx * ny);
-    return r;
-}
-
 // two floats as packed bf16 bits, the first in the low half
 __device__ __forceinline__ uint32_t pack_bf(float lo, float hi) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -844,12 +830,12 @@ __global__ __launch_bounds__(256) void kc_wgrad_first(int nx, int ny, int nz, lo
 }
 
 // bf16 weights of one layer: forward order wf[t][n][k] = W[t][n][k] and the
-// data-gradient order wb[t][k][n] = W[26 - t][n][k]
+// data-gradient order wb[t][k][n] = W[26 - t][n][k]; either may be NULL
 __device__ __forceinline__ void put_weight(int idx, float v, uint16_t *__restrict__ wf, uint16_t *__restrict__ wb) {
     const int t = idx / (C * C), n = (idx / C) % C, k = idx % C;
     const uint16_t h = f2bf(v);
-    wf[idx] = h;
-    wb[((size_t)(TAPS - 1 - t) * C + k) * C + n] = h;
+    if (wf) wf[idx] = h;
+    if (wb) wb[((size_t)(TAPS - 1 - t) * C + k) * C + n] = h;
 }
 
 __global__ void kc_prep_weights(const float *__restrict__ W, uint16_t *__restrict__ wf, uint16_t *__restrict__ wb) {

@@ -47,7 +47,7 @@ struct plsqr_cnn {
     uint16_t *dz[2] = {};             // gradients of the layers' outputs below
     float *wpart = nullptr, *bpart = nullptr, *lpart = nullptr;
     int *pick = nullptr;  // training pairs of loss_steps(max_batch) steps
-    float *xin = nullptr, *tgt = nullptr, *tn = nullptr, *x0 = nullptr;
+    float *xin = nullptr, *tgt = nullptr, *tn = nullptr;
     int count = 0;
     float *data_in = nullptr, *data_t = nullptr, *data_tn = nullptr;
     size_t data_bytes = 0;
@@ -390,17 +390,16 @@ int load_samples(plsqr_cnn *h, int batch, const double *atb, const double *xs, s
 
 // ---------------------------------------------------------------------------
 // Allocation-free variant of plsqr_cnn_conv_forward for callers that cannot
-// allocate device memory (HIP graph capture, serving loops): kc_conv rounds
-// the FP32 operands itself.  A call whose output overlaps its input or weights
-// needs copies of them first; that scratch -- the bf16 input and the two bf16
-// weight layouts -- lives in one file-scope device array, fixed in size; each
-// device holds its own copy, found once per device with hipGetSymbolAddress.
-// Every element the kernels read is written earlier in the same call, so no
-// clearing is needed; such calls that overlap on one device share the array
-// and race.
+// allocate device memory (HIP graph capture, serving loops): the layer kernels
+// round the FP32 operands themselves.  A call whose output overlaps its input or weights
+// needs copies of them first; that scratch -- the bf16 input and weights -- lives
+// in one file-scope device array, fixed in size; each device holds its own copy,
+// found once per device with hipGetSymbolAddress.  Every element the kernels read
+// is written earlier in the same call, so no clearing is needed; such calls that
+// overlap on one device share the array and race.
 // ---------------------------------------------------------------------------
 constexpr long long NOALLOC_MAX_ELEMS = 1LL << 22;  // batch * voxels * 32 channels of input
-constexpr size_t NOALLOC_BYTES = sizeof(uint16_t) * ((size_t)NOALLOC_MAX_ELEMS + 2 * (size_t)WSZ);
+constexpr size_t NOALLOC_BYTES = sizeof(uint16_t) * ((size_t)NOALLOC_MAX_ELEMS + (size_t)WSZ);
 static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
 
 namespace {
@@ -478,8 +477,7 @@ int plsqr_cnn_create(int nx, int ny, int nz, int max_batch, unsigned long long s
         (rc = calloc_dev(h, &h->wpart, (size_t)nch * TAPS * C * C)) || (rc = calloc_dev(h, &h->bpart, (size_t)nch * C)) ||
         (rc = calloc_dev(h, &h->lpart, (size_t)loss_steps(max_batch) * max_batch * LOSS_BLK)) ||
         (rc = calloc_dev(h, &h->pick, (size_t)loss_steps(max_batch) * max_batch)) || (rc = calloc_dev(h, &h->xin, (size_t)total)) ||
-        (rc = calloc_dev(h, &h->tgt, (size_t)total)) || (rc = calloc_dev(h, &h->tn, (size_t)max_batch)) ||
-        (rc = calloc_dev(h, &h->x0, (size_t)total)))
+        (rc = calloc_dev(h, &h->tgt, (size_t)total)) || (rc = calloc_dev(h, &h->tn, (size_t)max_batch)))
         return fail(rc);
     for (int l = 0; l < LAYERS; ++l)
         if ((rc = calloc_dev(h, &h->wf[l], WSZ)) || (rc = calloc_dev(h, &h->wb[l], WSZ)) ||
@@ -730,9 +728,9 @@ int plsqr_cnn_conv_forward_noalloc(int nx, int ny, int nz, int batch, const floa
         int rc = scratch_ptr(&base);
         if (rc) return rc;
         uint16_t *bin = (uint16_t *)base;
-        uint16_t *wf = bin + NOALLOC_MAX_ELEMS, *wb = wf + WSZ;
+        uint16_t *wf = bin + NOALLOC_MAX_ELEMS;
         hipLaunchKernelGGL(kc_to_bf16, dim3(grid_for(total * C, 256, 4096)), dim3(256), 0, st, total * C, in_dev, bin);
-        hipLaunchKernelGGL(kc_prep_weights, dim3((WSZ + 255) / 256), dim3(256), 0, st, w_dev, wf, wb);
+        hipLaunchKernelGGL(kc_prep_weights, dim3((WSZ + 255) / 256), dim3(256), 0, st, w_dev, wf, (uint16_t *)nullptr);
         conv<CONV_BF16, false, CONV_F32>(nx, ny, nz, batch, bin, wf, bias_dev, nullptr, relu, out_dev, st);
     }
     const hipError_t e = hipGetLastError();
@@ -749,7 +747,7 @@ int plsqr_cnn_conv_backward(int nx, int ny, int nz, int batch, const float *in, 
     const long long total = (long long)batch * nx * ny * nz;
     const int nch = (int)((total + WCHUNK - 1) / WCHUNK);
     float *fin = nullptr, *fw = nullptr, *fdo = nullptr, *fdi = nullptr, *gw = nullptr, *wpart = nullptr, *bpart = nullptr;
-    uint16_t *bin = nullptr, *bdo = nullptr, *wf = nullptr, *wb = nullptr;
+    uint16_t *bin = nullptr, *bdo = nullptr, *wb = nullptr;
     CallBuffers mem;
     mem.add(&fin, (size_t)total * C);
     mem.add(&fw, WSZ);
@@ -760,7 +758,6 @@ int plsqr_cnn_conv_backward(int nx, int ny, int nz, int batch, const float *in, 
     mem.add(&bpart, (size_t)nch * C);
     mem.add(&bin, (size_t)total * C);
     mem.add(&bdo, (size_t)total * C);
-    mem.add(&wf, WSZ);
     mem.add(&wb, WSZ);
     int rc;
     if ((rc = mem.alloc(g_cnn_err))) return rc;
@@ -771,7 +768,7 @@ int plsqr_cnn_conv_backward(int nx, int ny, int nz, int batch, const float *in, 
         const int g = grid_for(total * C, 256, 4096);
         hipLaunchKernelGGL(kc_to_bf16, dim3(g), dim3(256), 0, 0, total * C, (const float *)fin, bin);
         hipLaunchKernelGGL(kc_to_bf16, dim3(g), dim3(256), 0, 0, total * C, (const float *)fdo, bdo);
-        hipLaunchKernelGGL(kc_prep_weights, dim3((WSZ + 255) / 256), dim3(256), 0, 0, (const float *)fw, wf, wb);
+        hipLaunchKernelGGL(kc_prep_weights, dim3((WSZ + 255) / 256), dim3(256), 0, 0, (const float *)fw, (uint16_t *)nullptr, wb);
         conv<CONV_BF16, false, CONV_F32>(nx, ny, nz, batch, bdo, wb, nullptr, nullptr, 0, fdi, 0);
         rc = wgrad<false>(nullptr, nx, ny, nz, total, bin, bdo, gw, gw + WSZ, wpart, bpart, 0);
         e = hipGetLastError();
