@@ -78,6 +78,7 @@ struct plsqr_op {
     uint8_t *t_pvox = nullptr;
     long long *t_rbase = nullptr;
     int *t_roff = nullptr;
+    int place_rows = 0;  // rows up to which mode 1 updates a caller-order y in place
     bool nt_loads = false;
     int tw = 128;  // voxels per tile (brick) of the tiled layouts: 128 or 256
     bool rows_nt = false;  // streaming loads for the mode-1 matrix data
@@ -564,11 +565,14 @@ int b_internal(plsqr_op *op, const double *b, const double **out) {
     return PLSQR_OK;
 }
 
-// Rows up to which mode 1 updates a caller-order y in place.  The combine's
-// scattered 8 or 4 bytes per row cost more than two reordering passes once y is
-// far larger than the L2s (FP64 / FP32 mode 1 in us, in place against reordered:
-// 0.52M rows 60 / 43 against 71 / 52, 1.1M 148 / 94 against 158 / 105, 2.2M
-// 403 / 259 against 404 / 264, 3.2M 553 / 364 against 550 / 360).
+// Rows up to which mode 1 updates a caller-order y in place (PLSQR_IN_PLACE_ROWS).
+// It saves two passes over y, but the combine's scattered reads and writes, a
+// cache line per row whatever the element's width, hold up its other loads once
+// y has left the L2s.  FP64 / FP32 mode 1 in us, in place against reordered:
+// 0.55M rows 63 / 43 against 73 / 52, 1.1M 149 / 94 against 159 / 104, 2.3M
+// 378 / 246 against 378 / 250, 2.6M 486 / 313 against 488 / 314, 3.2M 555 / 365
+// against 552 / 361, 4.5M 941 / 609 against 939 / 592, 6.4M 1299 / 865 against
+// 1287 / 831.
 constexpr int IN_PLACE_ROWS = 2500000;
 
 // aprod on operands each either in the caller's order (renumbered in and,
@@ -578,7 +582,7 @@ int aprod_any(plsqr_op *op, int mode, double *x, bool x_ext, double *y, bool y_e
     int rc;
     const bool tiled = mode == 1 ? op->rtiled : op->tiled;
     const bool move_x = x_ext && op->permuted, move_y = y_ext && op->rowperm;
-    const bool place_x = mode == 2 && tiled && move_x, place_y = mode == 1 && tiled && move_y && op->m <= IN_PLACE_ROWS;
+    const bool place_x = mode == 2 && tiled && move_x, place_y = mode == 1 && tiled && move_y && op->m <= op->place_rows;
     double *xi = x, *yi = y;
     if (move_x && !place_x) {
         if ((rc = to_internal(op, x, op->hx2))) return rc;
@@ -1205,6 +1209,7 @@ int plsqr_op_create_ex(const plsqr_system *s, int flags, const plsqr_grid *grid,
         rays.reset();
     }
     // vectors and scratch
+    op->place_rows = env_int("PLSQR_IN_PLACE_ROWS", IN_PLACE_ROWS);
     op->nt_loads = env_int("PLSQR_NT", 0) != 0;
     op->rows_nt = env_int("PLSQR_ROWS_NT", 0) != 0;
     op->rt_lc = env_int("PLSQR_LC", 4);
@@ -1438,7 +1443,7 @@ int plsqr_aprod_device_f32(plsqr_op *op, int mode, float *x_dev, float *y_dev) {
     if ((rc = ensure_aprod32(op))) return rc;
     const int gn = grid_for(op->n, 256, op->cu * 4), gm = grid_for(op->m, 256, op->cu * 4);
     // caller order -> device order, except an output that a combine updates in place
-    const bool place_x = mode == 2 && op->permuted, place_y = mode == 1 && op->rowperm && op->rtiled && op->m <= IN_PLACE_ROWS;
+    const bool place_x = mode == 2 && op->permuted, place_y = mode == 1 && op->rowperm && op->rtiled && op->m <= op->place_rows;
     if (!place_x) {
         if (op->permuted)
             hipLaunchKernelGGL(k_gather32, dim3(gn), dim3(256), 0, op->stream, op->n, op->inv, x_dev, op->v32);
