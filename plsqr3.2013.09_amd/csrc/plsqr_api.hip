@@ -482,11 +482,22 @@ int launch_cols_exact(plsqr_op *op, const double *u, double *v, const Scal *sc) 
     return PLSQR_OK;
 }
 
+// Tile length of the exact order's sequential sums over vectors of at most len
+// elements.  A last tile is added whole, so up to half of a long one short ones
+// are faster (solves of 20 iterations in us, tiles of 512 / 64: 20 x 20 888 / 725,
+// 100 x 100 1010 / 851, 256 x 256 1085 / 953), and longer vectors pay for a
+// barrier per tile.
+constexpr int SEQ_TILE = 512, SEQ_TILE_SHORT = 64;
+bool short_tiles(int len) { return len <= SEQ_TILE / 2; }
+
 // the two halves of ||u|| (kernel rows, damping rows) side by side, and ||v||
 int launch_norms_exact(plsqr_op *op, const Scal *sc) {
     using namespace plsqr;
-    hipLaunchKernelGGL(k_dnrm2_seq, dim3(2), dim3(128), 0, op->stream, SeqVec{op->m_k, op->u, &op->sc->pk},
-                       SeqVec{op->m_d, op->u + op->m_k, &op->sc->pd}, sc, 0);
+    const SeqVec k{op->m_k, op->u, &op->sc->pk}, d{op->m_d, op->u + op->m_k, &op->sc->pd};
+    if (short_tiles(std::max(op->m_k, op->m_d)))
+        hipLaunchKernelGGL(k_dnrm2_seq<SEQ_TILE_SHORT>, dim3(2), dim3(128), 0, op->stream, k, d, sc, 0);
+    else
+        hipLaunchKernelGGL(k_dnrm2_seq<SEQ_TILE>, dim3(2), dim3(128), 0, op->stream, k, d, sc, 0);
     LAUNCH_CHECK(op);
     return PLSQR_OK;
 }
@@ -494,7 +505,10 @@ int launch_norms_exact(plsqr_op *op, const Scal *sc) {
 int launch_vnorm_exact(plsqr_op *op) {
     using namespace plsqr;
     const SeqVec v{op->n, op->v, &op->sc->pv};
-    hipLaunchKernelGGL(k_dnrm2_seq, dim3(1), dim3(128), 0, op->stream, v, v, (const Scal *)op->sc, 1);
+    if (short_tiles(op->n))
+        hipLaunchKernelGGL(k_dnrm2_seq<SEQ_TILE_SHORT>, dim3(1), dim3(128), 0, op->stream, v, v, (const Scal *)op->sc, 1);
+    else
+        hipLaunchKernelGGL(k_dnrm2_seq<SEQ_TILE>, dim3(1), dim3(128), 0, op->stream, v, v, (const Scal *)op->sc, 1);
     LAUNCH_CHECK(op);
     return PLSQR_OK;
 }
@@ -1617,7 +1631,10 @@ static int enqueue_iteration(plsqr_op *op, double *x, double *w, double *se, dou
         LAUNCH_CHECK(op);
         if ((rc = launch_cols_exact(op, op->u, op->v, op->sc)) || (rc = launch_vnorm_exact(op))) return rc;
         hipLaunchKernelGGL(k_s_alpha, dim3(1), dim3(256), 0, op->stream, op->sc, op->part, 0);
-        hipLaunchKernelGGL(k_dknorm_seq, dim3(1), dim3(128), 0, op->stream, op->n, w, op->sc);
+        if (short_tiles(op->n))
+            hipLaunchKernelGGL(k_dknorm_seq<SEQ_TILE_SHORT>, dim3(1), dim3(128), 0, op->stream, op->n, w, op->sc);
+        else
+            hipLaunchKernelGGL(k_dknorm_seq<SEQ_TILE>, dim3(1), dim3(128), 0, op->stream, op->n, w, op->sc);
         hipLaunchKernelGGL((k_update<BS>), dim3(op->G6), dim3(BS), 0, op->stream, op->n, (const Scal *)op->sc, op->v,
                            w, x, se, (double *)nullptr);
         LAUNCH_CHECK(op);

@@ -872,13 +872,11 @@ __global__ void k_scale_pending(long long len, const Scal *__restrict__ sc, doub
 // Sequential sums in the reference's order (exact-order mode only).  Every
 // addition depends on the one before it, so one FP64 add latency per element
 // is the floor; the terms do not, so a workgroup of two wavefronts splits the
-// work: one forms the terms of the next SEQ_T elements with coalesced loads
+// work: one forms the terms of the next T elements with coalesced loads
 // (the divisions of dnrm2 64 at a time), the other adds the tile before it
 // from LDS.  One lane doing both took 55 ns per element (a division and a
 // load on the chain), this 3.8 (dknorm) to 4.6 (dnrm2): the three norms of an
 // iteration at 24^3 / 60k rays 335 us, 17.0 ms before.
-constexpr int SEQ_T = 512;
-
 // acc += term[0..N) in order, all lanes alike (broadcast LDS reads, the next
 // sixteen terms read ahead of the additions of the sixteen before them)
 template <int N>
@@ -924,9 +922,10 @@ struct SeqVec {
 // larger), so the terms can be formed ahead; term[i] holds the squared
 // quotient, or scale/ax where bit i of `big` marks a new scale.  Zeros add
 // nothing (+0 to an ssq >= 1).
+template <int T>
 __global__ __launch_bounds__(128) void k_dnrm2_seq(SeqVec a, SeqVec b, const Scal *sc, int check_beta) {
-    __shared__ __align__(16) double term[2][SEQ_T];
-    __shared__ unsigned long long big[2][SEQ_T / kWave];
+    __shared__ __align__(16) double term[2][T];
+    __shared__ unsigned long long big[2][T / kWave];
     __shared__ double scale_end;
     if (sc && (sc->done || (check_beta && !sc->beta_pos))) return;  // uniform
     const SeqVec s = blockIdx.x == 0 ? a : b;
@@ -934,16 +933,16 @@ __global__ __launch_bounds__(128) void k_dnrm2_seq(SeqVec a, SeqVec b, const Sca
         if (threadIdx.x == 0) *s.out = s.len <= 0 ? 0.0 : fabs(s.v[0]);
         return;
     }
-    constexpr int NG = SEQ_T / kWave;
+    constexpr int NG = T / kWave;
     const int lane = threadIdx.x % kWave;
     const bool producer = threadIdx.x >= kWave;
-    const int tiles = (s.len + SEQ_T - 1) / SEQ_T;
+    const int tiles = (s.len + T - 1) / T;
     double scale = 0.0, ssq = 1.0;
     double x[NG];
     auto load = [&](int t) {
 #pragma unroll
         for (int g = 0; g < NG; ++g) {
-            x[g] = s.v[min((long long)t * SEQ_T + g * kWave + lane, (long long)s.len - 1)];
+            x[g] = s.v[min((long long)t * T + g * kWave + lane, (long long)s.len - 1)];
         }
     };
     if (producer) load(0);
@@ -951,7 +950,7 @@ __global__ __launch_bounds__(128) void k_dnrm2_seq(SeqVec a, SeqVec b, const Sca
         if (producer && t < tiles) {
 #pragma unroll
             for (int g = 0; g < NG; ++g) {
-                if ((long long)t * SEQ_T + g * kWave + lane >= s.len) x[g] = 0.0;
+                if ((long long)t * T + g * kWave + lane >= s.len) x[g] = 0.0;
                 const double ax = fabs(x[g]);
                 double before = scale;
                 unsigned long long mask = 0;
@@ -980,7 +979,7 @@ __global__ __launch_bounds__(128) void k_dnrm2_seq(SeqVec a, SeqVec b, const Sca
             unsigned long long any = 0;
 #pragma unroll
             for (int g = 0; g < NG; ++g) any |= big[(t - 1) & 1][g];
-            if (any == 0) ssq = seq_add<SEQ_T>(ssq, tt);
+            if (any == 0) ssq = seq_add<T>(ssq, tt);
             for (int g = 0; any != 0 && g < NG; ++g) {
                 const unsigned long long mask = big[(t - 1) & 1][g];
                 if (mask == 0) {
@@ -1000,31 +999,32 @@ __global__ __launch_bounds__(128) void k_dnrm2_seq(SeqVec a, SeqVec b, const Sca
 
 // dknorm of lsqr.c:685-690 in the reference's order: reads the w of before
 // the update.
+template <int T>
 __global__ __launch_bounds__(128) void k_dknorm_seq(int n, const double *__restrict__ w, Scal *sc) {
-    __shared__ __align__(16) double term[2][SEQ_T];
+    __shared__ __align__(16) double term[2][T];
     if (sc->done) return;  // uniform
     const double t3 = sc->t3;
     const int lane = threadIdx.x % kWave;
     const bool producer = threadIdx.x >= kWave;
-    const int tiles = (n + SEQ_T - 1) / SEQ_T;
+    const int tiles = (n + T - 1) / T;
     double dk = 0.0;
-    double x[SEQ_T / kWave];
+    double x[T / kWave];
     auto load = [&](int t) {
 #pragma unroll
-        for (int g = 0; g < SEQ_T / kWave; ++g)
-            x[g] = w[min((long long)t * SEQ_T + g * kWave + lane, (long long)n - 1)];
+        for (int g = 0; g < T / kWave; ++g)
+            x[g] = w[min((long long)t * T + g * kWave + lane, (long long)n - 1)];
     };
     if (producer) load(0);
     for (int t = 0; t <= tiles; ++t) {
         if (producer && t < tiles) {
 #pragma unroll
-            for (int g = 0; g < SEQ_T / kWave; ++g) {
-                const bool in = (long long)t * SEQ_T + g * kWave + lane < n;
+            for (int g = 0; g < T / kWave; ++g) {
+                const bool in = (long long)t * T + g * kWave + lane < n;
                 term[t & 1][g * kWave + lane] = in ? (t3 * x[g]) * (t3 * x[g]) : 0.0;
             }
             if (t + 1 < tiles) load(t + 1);
         } else if (threadIdx.x == 0 && t > 0) {
-            dk = seq_add<SEQ_T>(dk, term[(t - 1) & 1]);
+            dk = seq_add<T>(dk, term[(t - 1) & 1]);
         }
         __syncthreads();
     }
