@@ -869,14 +869,15 @@ __global__ void k_scale_pending(long long len, const Scal *__restrict__ sc, doub
         u[i] = u[i] * ib;
 }
 
-// Sequential sums in the reference's order (exact-order mode only).  Every
-// addition depends on the one before it, so one FP64 add latency per element
-// is the floor; the terms do not, so a workgroup of two wavefronts splits the
-// work: one forms the terms of the next T elements with coalesced loads
-// (the divisions of dnrm2 64 at a time), the other adds the tile before it
-// from LDS.  One lane doing both took 55 ns per element (a division and a
-// load on the chain), this 3.8 (dknorm) to 4.6 (dnrm2): the three norms of an
-// iteration at 24^3 / 60k rays 335 us, 17.0 ms before.
+// Sequential sums in the reference's order (exact-order mode only).  Added one
+// after another, as here, they take one FP64 add latency per element; the terms
+// do not depend on each other, so a workgroup of two wavefronts splits the work:
+// one forms the terms of the next T elements with coalesced loads (the divisions
+// of dnrm2 64 at a time), the other adds the tile before it from LDS.  24^3 / 60k
+// rays, per iteration: u's halves side by side (60,000 and 51,840 elements) 258 us,
+// v (13,824) 82 and dknorm (13,824) 53, 4.3, 5.9 and 3.8 ns per element.  One lane
+// doing both (a division and a load on the chain): 8180 + 7100, 1880 and 890 us,
+// 136 ns per element of dnrm2 and 64 of dknorm.
 // acc += term[0..N) in order, all lanes alike (broadcast LDS reads, the next
 // sixteen terms read ahead of the additions of the sixteen before them)
 template <int N>
