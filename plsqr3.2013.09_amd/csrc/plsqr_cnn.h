@@ -19,10 +19,6 @@
 // Weights are bf16 in [tap][out channel][in channel] order so that a lane's
 // eight k values are contiguous.  Tap t = (dz+1)*9 + (dy+1)*3 + (dx+1) reads
 // the neighbour at (x+dx, y+dy, z+dz); tap 26-t is its mirror.
-//
-// One 32x32x16 step adds its k = 0..7 and then its k = 8..15 exactly as two
-// 32x32x8 steps do (measured: no difference in 204,800 results over random
-// operands), at twice their rate, so results do not depend on which is used.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -70,11 +66,11 @@ __device__ __forceinline__ uint32_t pack_bf(float lo, float hi) {
 // and all weights lie in LDS, so each input row is read from memory about
 // twice instead of 27 times and the 27 taps are LDS reads at constant offsets
 // from one address per lane.  Wavefront w computes plane w of the brick as two
-// 32-voxel columns (8 x 4) that share each weight fragment.  With only
-// the LDS reads and matrix steps left the kernel takes 59 us of the 87 below, the rate a large matrix product reaches
-// here.  A voxel takes 80 bytes of LDS for its 64 and a line of voxels 896, so
-// that the 16-byte reads of 16 lanes (8 in x, 2 in y) fall on different banks
-// (with lines of 800 bytes half of the LDS cycles were conflicts: 118 us).  One
+// 32-voxel columns (8 x 4) that share each weight fragment.  With only the LDS
+// reads and matrix steps left the kernel takes 59 us of the 87 below (1.13
+// PFLOP/s; a large matrix product reaches 1.36).  A voxel takes 80 bytes of LDS
+// for its 64 and a line of voxels 896, so that the 16-byte reads of 16 lanes (8
+// in x, 2 in y) fall on different banks (with lines of 800 bytes half of the LDS cycles were conflicts: 118 us).  One
 // workgroup per CU stays for all of its bricks (weights are staged
 // once); the next brick's rows are loaded into registers while this one is
 // summed.  Workgroup b takes bricks of the b % 8-th of eight contiguous ranges,
@@ -519,7 +515,7 @@ __device__ __forceinline__ void bias_partial(float s, float *red, float *__restr
 // staged row's place took 112 of 200 vector instructions per 9 matrix steps,
 // 182 us; loading both operands two bytes at a time from memory, tap by tap,
 // took 1783 us.)
-// 67^3 x 4 samples: 136 us per layer.
+// 67^3 x 4 samples: 132 us per layer, 140 with a one-channel dout.
 //
 // Workgroup b works in the b % 8-th of eight contiguous ranges of chunks, so
 // the tap groups of a chunk and its neighbours share an XCD's L2.  The host
@@ -722,8 +718,8 @@ __global__ __launch_bounds__(GRAD_RED) void kc_grad_reduce(int nchunk, const flo
 // Per sub-block of 256 rows: dout, read transposed; for each (dz, dy) the 258
 // inputs its three taps read; and one byte per row that says which neighbours
 // exist.  Lane (tap t) gathers its eight rows' inputs from LDS; the next
-// sub-block's loads are in flight meanwhile.  67^3 x 4 samples: 44 us
-// (kc_wgrad on a 32-channel copy: 136, and 41 for the copy).
+// sub-block's loads are in flight meanwhile.  67^3 x 4 samples: 46 us
+// (kc_wgrad on a 32-channel copy: 132, and 41 for the copy).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void kc_wgrad_first(int nx, int ny, int nz, long long total, int chunk_len,
                                                       const float *__restrict__ x, const uint16_t *__restrict__ dout,
