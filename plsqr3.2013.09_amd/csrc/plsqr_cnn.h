@@ -567,9 +567,10 @@ __global__ __launch_bounds__(256, 2) void kc_wgrad(int nx, int ny, int nz, long 
                 ua[k] = ((const uint4_t *)dout + s * 4)[unit];
             if (tid + k * 256 >= live * 4) ua[k] = uint4_t{0, 0, 0, 0};
         }
-        // rows s + shift - halo .., clamped to the tensor (rows outside it are never used)
-        const long long r0 = s + shift - halo;
-        const int lo = (int)max(-r0, 0LL) * 4, hi = (int)max(min(total - r0, (long long)XROWS), 1 - r0) * 4 - 1;
+        // rows s + shift - halo .., clamped to the tensor (rows outside it are never
+        // used; a run wholly outside is moved to its end)
+        const long long r0 = min(max(s + shift - halo, 1LL - XROWS), total - 1);
+        const int lo = (int)max(-r0, 0LL) * 4, hi = (int)min(total - r0, (long long)XROWS) * 4 - 1;
         const uint4_t *from = (const uint4_t *)in + r0 * 4;
 #pragma unroll
         for (int k = 0; k < PX; ++k)

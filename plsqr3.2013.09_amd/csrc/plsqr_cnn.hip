@@ -221,7 +221,9 @@ void conv(int nx, int ny, int nz, int samples, const void *in, const void *w, co
     const long long tiles = bricks(nx) * bricks(ny) * bricks(nz) * samples, rows = (long long)nx * ny * nz * samples;
     const int aligned = (((uintptr_t)in | (uintptr_t)out) & 15) == 0, cus = compute_units();
     const long long brick_rounds = (tiles + cus - 1) / cus, row_blocks = (rows + 32 * CB - 1) / (32 * CB);
-    if (brick_rounds > 2 * ((row_blocks + cus - 1) / cus)) {
+    // the offsets within a brick's neighbourhood have 32 bits
+    const bool wide = (long long)CH * nx * ny * 4 > UINT32_MAX;
+    if (wide || brick_rounds > 2 * ((row_blocks + cus - 1) / cus)) {
         const long long g = std::min<long long>(row_blocks, cus);
         hipLaunchKernelGGL((kc_conv_rows<IN, WF32, OUT>), dim3((unsigned)g), dim3(CONV_THREADS), 0, st, nx, ny, nz, (unsigned)rows,
                            in, w, bias, mask, relu, out, aligned);
